@@ -62,6 +62,17 @@ __device__ __forceinline__ uint16_t f32_to_f16_bits(float f) {
   return b;
 }
 
+// Two floats rounded to nearest-even to a pair of bf16 (one v_cvt_pk_bf16_f32)
+// or fp16 values, the first in the low half.
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(lo), static_cast<__bf16>(hi)});
+}
+__device__ __forceinline__ uint32_t pack_f16(float lo, float hi) {
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, f16x2{static_cast<_Float16>(lo), static_cast<_Float16>(hi)});
+}
+
 // Element i of an fp32 / fp16 / bf16 array, in two parts so that a caller can
 // issue the load early and convert where the value is used: elem_word loads
 // the aligned 32-bit word that holds the element (a 16-bit element is its low

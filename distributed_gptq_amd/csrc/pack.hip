@@ -118,71 +118,93 @@ __global__ void dequant_k(const uint8_t* __restrict__ packed, int bits, const vo
   }
 }
 
-template <int BITS, int PP>
-__device__ __forceinline__ void dequant_pair(const uint32_t (&w)[BITS], float z, float s, float (&v)[32]) {
-  const uint32_t cp = chunk_pair<BITS, PP>(w);
-  const float d0 = static_cast<float>(cp & 0xFFFFu) - z, d1 = static_cast<float>(cp >> 16) - z;
-  v[2 * PP] = d0 * s;
-  v[2 * PP + 1] = d1 * s;
-}
-template <int BITS, int... PP>
-__device__ __forceinline__ void dequant_pairs(const uint32_t (&w)[BITS], float z, float s, float (&v)[32],
-                                              std::integer_sequence<int, PP...>) {
-  (dequant_pair<BITS, PP>(w, z, s, v), ...);
-}
+// The same for K % 32 == 0 and groups of a multiple of 32 columns.  Bound by
+// the stores: a thread takes 8 codes of kDqRows rows, so that a wave's store
+// is 1 KB of consecutive bytes (16-bit outputs; with 32 codes a thread the
+// four 16-byte stores were 64 bytes apart between lanes and 28672 x 4096 to
+// bf16 took 94 us against 57, 297 MB moved), and the loads of all rows
+// are in flight together.
+constexpr int kDqRows = 4;
 
-// The same for K % 32 == 0 and groups of a multiple of 32 columns: one thread
-// per 32-code chunk (one group), one 4 * BITS-byte load and 64 (128 for fp32)
-// contiguous bytes stored; consecutive threads take consecutive chunks.
-template <int BITS>
-__global__ __launch_bounds__(256) void dequant_chunks_k(const uint8_t* __restrict__ packed,
-                                                        const void* __restrict__ scales,
-                                                        const void* __restrict__ zeros, int sz_dtype, int gs,
-                                                        int64_t ngroups, int64_t N, int64_t nch, int64_t pitch,
-                                                        void* __restrict__ out, int out_dtype) {
-  const int64_t total = N * nch;
-  for (int64_t idx = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; idx < total;
-       idx += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int64_t n = idx / nch, c = idx - n * nch;
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(packed + n * pitch + c * 4 * BITS);
-    uint32_t w[BITS];
-    if constexpr (BITS == 4) {
-      const uint4 v = *reinterpret_cast<const uint4*>(src);
-      w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
-    } else if constexpr (BITS == 8) {
-      const uint4 v0 = reinterpret_cast<const uint4*>(src)[0], v1 = reinterpret_cast<const uint4*>(src)[1];
-      w[0] = v0.x; w[1] = v0.y; w[2] = v0.z; w[3] = v0.w; w[4] = v1.x; w[5] = v1.y; w[6] = v1.z; w[7] = v1.w;
-    } else if constexpr (BITS == 2) {
-      const uint2 v = *reinterpret_cast<const uint2*>(src);
-      w[0] = v.x; w[1] = v.y;
-    } else {
-      w[0] = src[0]; w[1] = src[1]; w[2] = src[2];
-    }
-    const int64_t g = (c * 32) / gs;
-    const float z = load_elem(zeros, n * ngroups + g, sz_dtype);
-    const float s = load_elem(scales, n * ngroups + g, sz_dtype);
-    float v[32];
-    dequant_pairs<BITS>(w, z, s, v, std::make_integer_sequence<int, 16>{});
-    if (out_dtype == GPTQ_F32) {
-      uint4* dst = reinterpret_cast<uint4*>(static_cast<float*>(out) + idx * 32);
+template <int BITS, int OUT>
+__global__ __launch_bounds__(256) void dequant_rows_k(const uint8_t* __restrict__ packed,
+                                                      const void* __restrict__ scales,
+                                                      const void* __restrict__ zeros, int sz_dtype, int gs,
+                                                      int64_t ngroups, int64_t N, int64_t n8, int64_t pitch,
+                                                      void* __restrict__ out) {
+  const int64_t c = blockIdx.x * 256LL + threadIdx.x;
+  if (c >= n8) return;
+  const int g = static_cast<int>(c * 8) / gs;
+  for (int64_t n0 = static_cast<int64_t>(blockIdx.y) * kDqRows; n0 < N; n0 += static_cast<int64_t>(gridDim.y) * kDqRows) {
+    uint32_t w[kDqRows][2];
+    uint32_t zw[kDqRows], sw[kDqRows];
+    bool zh[kDqRows], sh[kDqRows];
 #pragma unroll
-      for (int q = 0; q < 8; ++q)
-        dst[q] = uint4{__float_as_uint(v[4 * q]), __float_as_uint(v[4 * q + 1]), __float_as_uint(v[4 * q + 2]),
-                       __float_as_uint(v[4 * q + 3])};
-    } else {
-      const bool bf = out_dtype == GPTQ_BF16;
-      uint32_t h[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const uint32_t lo = bf ? f32_to_bf16_bits(v[2 * q]) : f32_to_f16_bits(v[2 * q]);
-        const uint32_t hi = bf ? f32_to_bf16_bits(v[2 * q + 1]) : f32_to_f16_bits(v[2 * q + 1]);
-        h[q] = lo | (hi << 16);
+    for (int r = 0; r < kDqRows; ++r) {
+      const int64_t n = n0 + r < N ? n0 + r : N - 1;
+      const uint8_t* row = packed + n * pitch;
+      if constexpr (BITS == 4) {
+        w[r][0] = *reinterpret_cast<const uint32_t*>(row + c * 4);
+      } else if constexpr (BITS == 8) {
+        const uint2 v = *reinterpret_cast<const uint2*>(row + c * 8);
+        w[r][0] = v.x;
+        w[r][1] = v.y;
+      } else if constexpr (BITS == 2) {
+        w[r][0] = *reinterpret_cast<const uint16_t*>(row + c * 2);
+      } else {
+        // 24 bits at byte 3c: the two words that hold them (the row is a multiple of 12 bytes)
+        const int64_t d = (c * 3) >> 2, last = (pitch >> 2) - 1;
+        w[r][0] = reinterpret_cast<const uint32_t*>(row)[d];
+        w[r][1] = reinterpret_cast<const uint32_t*>(row)[d < last ? d + 1 : last];
       }
-      uint4* dst = reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + idx * 32);
+      zw[r] = elem_word(zeros, n * ngroups + g, sz_dtype, zh[r]);
+      sw[r] = elem_word(scales, n * ngroups + g, sz_dtype, sh[r]);
+    }
 #pragma unroll
-      for (int q = 0; q < 4; ++q) dst[q] = uint4{h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]};
+    for (int r = 0; r < kDqRows; ++r) {
+      if (n0 + r >= N) break;
+      const float z = elem_value(zw[r], zh[r], sz_dtype), s = elem_value(sw[r], sh[r], sz_dtype);
+      uint32_t bits = w[r][0];
+      if constexpr (BITS == 3) bits = __builtin_amdgcn_alignbyte(w[r][1], w[r][0], static_cast<uint32_t>(c * 3) & 3u);
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t q = BITS == 8 ? (w[r][e / 4] >> (8 * (e & 3))) & 0xFFu : (bits >> (BITS * e)) & ((1u << BITS) - 1);
+        const float d = static_cast<float>(q) - z;
+        v[e] = d * s;
+      }
+      const int64_t at = (n0 + r) * n8 + c;
+      if constexpr (OUT == GPTQ_F32) {
+        f32x4* dst = reinterpret_cast<f32x4*>(out) + at * 2;
+        dst[0] = f32x4{v[0], v[1], v[2], v[3]};
+        dst[1] = f32x4{v[4], v[5], v[6], v[7]};
+      } else {
+        u32x4 h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          h[e] = OUT == GPTQ_BF16 ? pack_bf16(v[2 * e], v[2 * e + 1]) : pack_f16(v[2 * e], v[2 * e + 1]);
+        reinterpret_cast<u32x4*>(out)[at] = h;
+      }
     }
   }
+}
+
+template <int BITS>
+void launch_dequant_rows(const uint8_t* packed, const void* scales, const void* zeros, int sz_dtype, int gs,
+                         int64_t ngroups, int64_t N, int64_t K, int64_t pitch, void* out, int out_dtype,
+                         hipStream_t st) {
+  const int64_t n8 = K / 8;
+  const dim3 grid(static_cast<unsigned>(cdiv(n8, 256)),
+                  static_cast<unsigned>(std::min<int64_t>(cdiv(N, kDqRows), 65535)));
+  if (out_dtype == GPTQ_F32)
+    hipLaunchKernelGGL((dequant_rows_k<BITS, GPTQ_F32>), grid, dim3(256), 0, st, packed, scales, zeros, sz_dtype, gs,
+                       ngroups, N, n8, pitch, out);
+  else if (out_dtype == GPTQ_BF16)
+    hipLaunchKernelGGL((dequant_rows_k<BITS, GPTQ_BF16>), grid, dim3(256), 0, st, packed, scales, zeros, sz_dtype, gs,
+                       ngroups, N, n8, pitch, out);
+  else
+    hipLaunchKernelGGL((dequant_rows_k<BITS, GPTQ_F16>), grid, dim3(256), 0, st, packed, scales, zeros, sz_dtype, gs,
+                       ngroups, N, n8, pitch, out);
 }
 
 // -------------------------------------------------- flat tensor quantiser --
@@ -299,18 +321,12 @@ extern "C" int gptq_dequant_to(const uint8_t* packed, int bits, const void* scal
   const int64_t pitch = bits == 0 ? K : pitch_of(K, bits);
   hipStream_t st = as_hip(stream);
   const bool aligned = (reinterpret_cast<uintptr_t>(packed) % 16) == 0 && (reinterpret_cast<uintptr_t>(out) % 16) == 0;
-  if (!g_idx && bits != 0 && K % 32 == 0 && group_size % 32 == 0 && aligned) {
-    const int64_t nch = K / 32;
-    const unsigned blocks = static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>(cdiv(N * nch, 256), 16384)));
+  if (!g_idx && bits != 0 && K % 32 == 0 && K < (int64_t(1) << 31) && group_size % 32 == 0 && aligned) {
     switch (bits) {
-      case 4: hipLaunchKernelGGL(dequant_chunks_k<4>, dim3(blocks), dim3(256), 0, st, packed, scales, zeros, sz_dtype,
-                                 group_size, ngroups, N, nch, pitch, out, out_dtype); break;
-      case 3: hipLaunchKernelGGL(dequant_chunks_k<3>, dim3(blocks), dim3(256), 0, st, packed, scales, zeros, sz_dtype,
-                                 group_size, ngroups, N, nch, pitch, out, out_dtype); break;
-      case 2: hipLaunchKernelGGL(dequant_chunks_k<2>, dim3(blocks), dim3(256), 0, st, packed, scales, zeros, sz_dtype,
-                                 group_size, ngroups, N, nch, pitch, out, out_dtype); break;
-      default: hipLaunchKernelGGL(dequant_chunks_k<8>, dim3(blocks), dim3(256), 0, st, packed, scales, zeros,
-                                  sz_dtype, group_size, ngroups, N, nch, pitch, out, out_dtype); break;
+      case 4: launch_dequant_rows<4>(packed, scales, zeros, sz_dtype, group_size, ngroups, N, K, pitch, out, out_dtype, st); break;
+      case 3: launch_dequant_rows<3>(packed, scales, zeros, sz_dtype, group_size, ngroups, N, K, pitch, out, out_dtype, st); break;
+      case 2: launch_dequant_rows<2>(packed, scales, zeros, sz_dtype, group_size, ngroups, N, K, pitch, out, out_dtype, st); break;
+      default: launch_dequant_rows<8>(packed, scales, zeros, sz_dtype, group_size, ngroups, N, K, pitch, out, out_dtype, st); break;
     }
     return check_launch("dequant");
   }
