@@ -53,6 +53,9 @@ SIGNATURES = {
     "gptq_pack_reference_layout": (_i, [_p, _i64, _i64, _i, _p, _p]),
     "gptq_dequant": (_i, [_p, _i, _p, _p, _i, _p, _i, _i64, _i64, _i64, _p, _p]),
     "gptq_dequant_to": (_i, [_p, _i, _p, _p, _i, _p, _i, _i64, _i64, _i64, _p, _i, _p]),
+    "gptq_dequant_planes_t": (_i, [_p, _i, _p, _p, _i, _i, _i64, _i64, _i64, _p, _p, _p, _p]),
+    "gptq_split_planes": (_i, [_p, _i64, _i64, _p, _p]),
+    "gptq_matmul_nt": (_i, [_p, _i64, _p, _i64, _i, _i64, _i64, _i64, _i, _i, _p, _p, _i, _p, _i64, _i, _p]),
     "gptq_linear": (_i, [_p, _i, _i64, _p, _i, _p, _p, _i, _p, _i, _i64, _p, _i, _i64, _i64, _p, _p]),
     "gptq_linear_perm_workspace_size": (_sz, [_i64, _i64, _i]),
     "gptq_linear_workspace_size": (_sz, [_i64, _i64, _i64, _i, _i, _i, _i]),

@@ -268,6 +268,56 @@ def dequant(packed: torch.Tensor, bits: int, scales: torch.Tensor, zeros: torch.
     return out
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """``t`` contiguous, its first element on a 16-byte boundary."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def matmul_nt(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """y = x @ W^T (+ bias) for 16-bit x (M, K) and W (N, K) of one dtype:
+    fp32 sums, one rounding to x's dtype."""
+    _gpu(x, W)
+    x, W = _aligned(x), _aligned(W)
+    M, K = x.shape
+    N = W.shape[0]
+    if bias is not None:
+        bias = bias.contiguous()
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    L.call("gptq_matmul_nt", _p(x), K, _p(W), K, dtype_code(x.dtype), M, N, K, 1, 1, _p(None), _p(bias),
+           dtype_code(bias.dtype) if bias is not None else 0, _p(y), N, dtype_code(y.dtype), _stream(x.device))
+    return y
+
+
+def linear_grad_input(grad: torch.Tensor, packed: torch.Tensor, bits: int, scales: torch.Tensor,
+                      zeros: torch.Tensor, K: int, group_size: int, perm: torch.Tensor | None = None) -> torch.Tensor:
+    """grad (M, N) @ dequant(W) (N, K; input-column order) in grad's 16-bit
+    dtype.  The fp32 weights are split exactly into bf16 planes (and an fp16
+    grad into two), whose products are summed in fp32."""
+    _gpu(grad, packed, scales, zeros)
+    packed, scales = _aligned(packed), scales.contiguous()
+    zeros = zeros.to(scales.dtype).contiguous()
+    grad = _aligned(grad)
+    M, N = grad.shape
+    dev, st = grad.device, _stream(grad.device)
+    if perm is not None:
+        perm = perm.to(device=dev, dtype=torch.int32).contiguous()
+        if perm.numel() != K:
+            raise ValueError(f"perm has {perm.numel()} entries, in_features is {K}")
+    planes = torch.empty((K, 3 * N), dtype=torch.bfloat16, device=dev)
+    flags = torch.empty(256, dtype=torch.int32, device=dev)
+    L.call("gptq_dequant_planes_t", _p(packed), bits, _p(scales), _p(zeros), dtype_code(scales.dtype), group_size,
+           scales.shape[1], N, K, _p(perm), _p(flags), _p(planes), st)
+    a, ap = grad, 1
+    if grad.dtype == torch.float16:
+        a, ap = torch.empty((M, 2 * N), dtype=torch.bfloat16, device=dev), 2
+        L.call("gptq_split_planes", _p(grad), M, N, _p(a), st)
+    gx = torch.empty((M, K), dtype=grad.dtype, device=dev)
+    L.call("gptq_matmul_nt", _p(a), ap * N, _p(planes), 3 * N, L.BF16, M, K, N, ap, 3, _p(flags), _p(None), 0,
+           _p(gx), K, dtype_code(gx.dtype), st)
+    return gx
+
+
 def linear(x: torch.Tensor, packed: torch.Tensor, bits: int, scales: torch.Tensor, zeros: torch.Tensor, K: int,
            g_idx: torch.Tensor | None = None, group_size: int = 0, bias: torch.Tensor | None = None,
            out: torch.Tensor | None = None, perm: torch.Tensor | None = None) -> torch.Tensor:

@@ -26,7 +26,7 @@
 // token-major LDS tile (no transpose needed).
 #include <type_traits>
 
-#include "common.hpp"
+#include "mfma_lds.hpp"
 
 namespace gptq {
 namespace {
@@ -334,7 +334,6 @@ __device__ __forceinline__ int dma_sig(int r) { return 10 * (r & 1) + 4 * ((r >>
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-typedef __attribute__((address_space(3))) void lds_void;
 
 __device__ __forceinline__ u32x4 tr_frag(const uint8_t* p) {
   // (generic -> LDS address-space casts have to be C-style)
@@ -357,52 +356,6 @@ __shared__ __attribute__((aligned(1024))) uint8_t g_hslab2[2][kStageB];
 template <int B>
 __device__ __forceinline__ uint8_t* hslab(int op) {
   return B == 0 ? &g_hslab0[op][0] : B == 1 ? &g_hslab1[op][0] : &g_hslab2[op][0];
-}
-
-template <bool kBF16>
-__device__ __forceinline__ void mfma32_asm(f32x16& acc, const u32x4& a, const u32x4& b) {
-  if constexpr (kBF16)
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-  else
-    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-}
-
-// A wave-uniform 64-bit value through readfirstlane, which takes and returns
-// int: each half is widened as unsigned, so that a low half with bit 31 set
-// does not sign-extend into the high half.
-__device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
-  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(v))));
-  const uint32_t hi =
-      static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(v >> 32))));
-  return static_cast<uint64_t>(hi) << 32 | lo;
-}
-
-// One 16-byte-per-lane copy into LDS from base + voff, zeros at and past nrec
-// bytes.  base and nrec are wave-uniform (the descriptor stays in SGPRs).
-// (Target builtins sit in a __device__ function, not in the kernel body: in
-// the kernel body the host pass dropped the kernel's launch stub.)
-__device__ __forceinline__ void lds_copy16(const uint16_t* base, uint32_t nrec, uint8_t* lds, uint32_t voff) {
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-      reinterpret_cast<uint16_t*>(uniform_u64(reinterpret_cast<uint64_t>(base))), static_cast<short>(0),
-      __builtin_amdgcn_readfirstlane(static_cast<int>(nrec)), 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)lds, 16, voff, 0, 0, 0);
-}
-
-__device__ __forceinline__ void bare_barrier() { asm volatile("s_barrier" ::: "memory"); }
-
-// s_waitcnt for "at most N vector-memory operations outstanding" (gfx9
-// encoding: vmcnt bits 3:0 and 15:14; expcnt and lgkmcnt left at "no wait")
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N < 64, "vmcnt immediate");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
-
-// s_waitcnt for "at most N LDS / scalar-memory operations outstanding"
-template <int N>
-__device__ __forceinline__ void wait_lgkm() {
-  static_assert(N < 16, "lgkmcnt immediate");
-  __builtin_amdgcn_s_waitcnt(0xC07F | (N << 8));
 }
 
 // copy slots: after which MFMA m of a step the step's j-th copy goes (-1:
@@ -586,9 +539,7 @@ void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ld
     }
     // no copy may still be writing LDS when the workgroup ends
     wait_vm<0>();
-    // the accumulators are read below: wait states after the last MFMA (the
-    // compiler does not see the asm MFMAs' results as MFMA results)
-    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+    mfma_settle();  // the accumulators are read below
   }
 
   // 32x32 accumulator layout: lane l, register v -> row 8*(v/4) + 4*(l/32) + v%4, col l%32

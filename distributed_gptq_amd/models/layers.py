@@ -156,6 +156,46 @@ def _gather_code_columns(qweight: torch.Tensor, bits: int, packed: bool, K: int,
     return _pack_rows(_unpack_rows(qweight, bits, K)[:, idx], bits)
 
 
+def _dense_rounds(M: int, N: int) -> float:
+    """Rounds of the GPU's 256 compute units that the dense kernel's 256 x 256
+    tiles of an (M, N) product take; a last round of at most 128 tiles runs as
+    halves, in 0.55 of a round."""
+    full, rest = divmod(-(-M // 256) * -(-N // 256), 256)
+    return full + (0.55 if 0 < rest <= 128 else 1.0 if rest else 0.0)
+
+
+def _dense_forward(M: int, N: int, K: int) -> bool:
+    """Whether x @ W^T on many rows runs on the dense kernel: where its tiles
+    fill at least 65% of the rounds they take.  Measured (bf16, us, against
+    the library GEMM with fp32 output and the cast; M, N, K): 2048 x 28672 x
+    4096 (0.88 filled) 415 / 565, 512 x 28672 x 4096 (0.88) 88 / 118, 2048 x
+    4096 x 4096 (0.91) 58 / 72; below, 2048 x 5120 x 5120 (0.63) 108 / 101,
+    1024 x 4096 x 14336 (0.45) 157 / 120."""
+    if K % 64 or N % 8 or max(M, N) > 1 << 24 or K >= 1 << 22:  # the kernel's ranges
+        return False
+    return M * N >= 0.65 * _dense_rounds(M, N) * 256 * 65536
+
+
+def _planes_backward(M: int, N: int, K: int, bits: int, dtype: torch.dtype, perm) -> bool:
+    """Whether grad @ W runs on the weight's bf16 planes instead of the fp32
+    library product: by the two sides' times on MI355X.  A stage of 64 of the
+    contraction takes the dense kernel 1.5 us a round (0.7 us a round of
+    halves); codes of up to 4 bits take 2 planes, 8-bit codes 3, an fp16 grad
+    twice that; the fp32 product runs at 130 TFLOP/s, and putting an act-order
+    weight into input order costs it 8 us per million weights.  Measured (4-bit
+    bf16, us, new / old): 4096 x 14336 M = 64 / 256 / 1024: 193 / 215 / 266
+    against 149 / 317 / 908; 8-bit 14336 x 4096 M = 512 / 1024: 625 / 625
+    against 589 / 967."""
+    if N % 64 or K % 32 or max(M, K) > 1 << 24 or N > 1 << 20:  # the kernels' ranges
+        return False
+    rounds = _dense_rounds(M, K)
+    half = 0.7 if rounds % 1 else 0.0
+    planes = (2 if 0 < bits <= 4 else 3) * (2 if dtype == torch.float16 else 1)
+    new = planes * N / 64 * (1.5 * int(rounds) + half)
+    old = M * N * K / 65e6 + (8e-6 * N * K if perm is not None else 0.0)
+    return new < old
+
+
 def _linear_impl(x, qweight, scales, zeros, g_idx, bias, perm=None):
     K = g_idx.numel()
     bits = _infer_bits(qweight, K)
@@ -178,6 +218,8 @@ def _linear_impl(x, qweight, scales, zeros, g_idx, bias, perm=None):
         # x's dtype (a 16-bit product may otherwise reduce split-K partials in
         # 16 bits, torch's allow_*_reduced_precision_reduction default)
         x2 = x.reshape(-1, K)
+        if _dense_forward(rows, W.shape[0], K):
+            return _ops.matmul_nt(x2, W, bias).reshape(*x.shape[:-1], W.shape[0])
         if bias is None:
             y = torch.mm(x2, W.t(), out_dtype=torch.float32)
         else:
@@ -207,14 +249,33 @@ def _linear_setup(ctx, inputs, output):
     ctx.has_bias = bias is not None
 
 
+def _grad_input(grad, qweight, scales, zeros, g_idx, perm, dtype) -> torch.Tensor:
+    """grad @ W in ``dtype``, W the fp32 dequantised weights."""
+    N, K = qweight.shape[0], g_idx.numel()
+    M = grad.numel() // N if N else 0
+    # (a grad that is itself differentiated, or a wrapper without storage as
+    # under vmap, takes the torch product)
+    plain = type(grad) is torch.Tensor and torch._C._has_storage(grad) and not (
+        torch._C._functorch.is_functorch_wrapped_tensor(grad) or (torch.is_grad_enabled() and grad.requires_grad))
+    if M and plain and grad.dtype == dtype and dtype in (torch.float16, torch.bfloat16):
+        order = perm if perm is not None and perm.numel() else None
+        bits = _infer_bits(qweight, K)
+        if _planes_backward(M, N, K, bits, dtype, order):
+            gs, gi = _group_layout(g_idx, K, scales.shape[1], order)
+            if gi is None and gs % 32 == 0 and qweight.contiguous().data_ptr() % 16 == 0:
+                gx = _ops.linear_grad_input(grad.reshape(M, N), qweight, bits, scales, zeros, K, gs, order)
+                return gx.reshape(*grad.shape[:-1], K)
+    W = _dequant_input_order(qweight, scales, zeros, g_idx, perm)
+    return (grad.float() @ W).to(dtype)
+
+
 def _linear_backward(ctx, grad):
     """Gradients of the fallback F.linear(x, unpack_weights(), bias): the
     quantized weights are constants; x and bias get their usual gradients."""
     qweight, scales, zeros, g_idx, perm = ctx.saved_tensors
     gx = gb = None
     if ctx.needs_input_grad[0]:
-        W = _dequant_input_order(qweight, scales, zeros, g_idx, perm)
-        gx = (grad.float() @ W).to(ctx.x_dtype)
+        gx = _grad_input(grad, qweight, scales, zeros, g_idx, perm, ctx.x_dtype)
     if ctx.has_bias and ctx.needs_input_grad[5]:
         gb = grad.reshape(-1, grad.shape[-1]).float().sum(0)
     return gx, None, None, None, None, gb, None

@@ -283,6 +283,41 @@ int gptq_linear_perm_noalloc(const void* x, int x_dtype, int64_t M,
                              int bias_dtype, int64_t N, int64_t K, void* y,
                              gptq_stream_t stream);
 
+/* -------------------------------------------------------- dense products --
+ * C = A B^T (+ bias) on bf16 / fp16 MFMA, fp32 accumulation, one rounding to
+ * out_dtype: A (M x K, row stride lda elements), B (N x K, ldb), both with the
+ * contraction contiguous and 16-byte aligned rows, C (M x N, ldc), bias N
+ * values or NULL.  K % 64 == 0, N % 8 == 0.  Used for
+ * F.linear(x, unpack_weights(), bias) (models/layers.py:155-157) on many rows.
+ *
+ * With planes, A and B are bf16 and hold `aplanes` (1 or 2) and 3 matrices of
+ * K columns side by side; every plane of A meets every plane of B.  `inexact`
+ * (256 ints, from gptq_dequant_planes_t) tells the kernel whether B's third
+ * plane is used; results that come out infinite or NaN are summed again term
+ * by term, as the unsplit product would. */
+int gptq_matmul_nt(const void* A, int64_t lda, const void* B, int64_t ldb,
+                   int dtype, int64_t M, int64_t N, int64_t K, int aplanes,
+                   int bplanes, const int32_t* inexact, const void* bias,
+                   int bias_dtype, void* C, int64_t ldc, int out_dtype,
+                   gptq_stream_t stream);
+
+/* The weights of gptq_dequant (contiguous groups of group_size columns; bits
+ * 0: one code per byte) transposed and split exactly into three bf16 planes:
+ * out row k (row perm[k] with perm) holds column k's N weights three times,
+ * 3 N values.  N % 64 == 0, K % 32 == 0, group_size % 32 == 0, packed and out
+ * 16-byte aligned.  flags (256 ints) are written: all zero when two planes
+ * hold every weight, the third then is not written.  For the input gradient
+ * of F.linear(x, unpack_weights()) (models/layers.py:155-157). */
+int gptq_dequant_planes_t(const uint8_t* packed, int bits, const void* scales,
+                          const void* zeros, int sz_dtype, int group_size,
+                          int64_t ngroups, int64_t N, int64_t K,
+                          const int32_t* perm, int32_t* flags, void* out,
+                          gptq_stream_t stream);
+
+/* fp16 (M x N, contiguous, N % 8 == 0) -> its two bf16 planes, M x 2N. */
+int gptq_split_planes(const void* x, int64_t M, int64_t N, void* out,
+                      gptq_stream_t stream);
+
 /* ------------------------------------------------- elementwise quantise --
  * Flat groups of group_size consecutive elements (the tensor API of
  * kernels/triton_kernels.py:377-481): per group s = (max - min) / maxq,

@@ -1,10 +1,147 @@
-"""The row-wise dequantisation at the edges of its workgroups, against the
-formula."""
+"""The dense MFMA product, the transposed weight planes and the row-wise
+dequantisation, at the edges of their tiles, against fp64."""
 import numpy as np
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float16, torch.bfloat16]
+
+
+def half_ulp(ref, dtype):
+    """Half a unit in the last place of ``dtype`` at |ref| (fp64)."""
+    p, emin = (11, -14) if dtype == torch.float16 else (8, -126)
+    e = torch.floor(torch.log2(ref.abs().clamp(min=2.0 ** emin))).clamp(min=emin)
+    return torch.exp2(e - p)
+
+
+def check(y, ref, mag, depth):
+    """|y - ref| within half an ulp of y's type plus the worst case of an fp32
+    sum of ``depth`` roundings over terms of total magnitude ``mag``."""
+    acc = depth * 2.0 ** -24 * mag
+    bound = half_ulp(ref.abs() + acc, y.dtype) + acc
+    worst = ((y.double() - ref).abs() / bound).max().item()
+    assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("M,N,K", [
+    (1, 8, 64),           # one row, the smallest N and K
+    (255, 136, 128),      # inside one half tile and past it
+    (257, 264, 192),      # one row and one chunk into the next tiles, an odd stage count
+    (513, 1000, 4096),
+    (4096, 4096, 64),     # 256 whole tiles
+    (4300, 4096, 128),    # a whole round and 16 tiles as halves
+    (6200, 4104, 64),     # a whole round and more than 128 tiles
+])
+def test_matmul_nt(M, N, K, dtype):
+    from distributed_gptq_amd import _ops
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).to(dtype)
+    bias = torch.randn(N, generator=g, device="cuda")
+    xd, wd = x.double(), w.double()
+    ref, mag = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    check(_ops.matmul_nt(x, w), ref, mag, K)
+    for b in (bias, bias.to(dtype)):
+        check(_ops.matmul_nt(x, w, b), ref + b.double(), mag + b.double().abs(), K + 1)
+
+
+def test_matmul_nt_misaligned_and_strided():
+    from distributed_gptq_amd import _ops
+    g = torch.Generator(device="cuda").manual_seed(1)
+    flat = torch.randn(300 * 64 + 1, generator=g, device="cuda").half()
+    w = torch.randn(64, 72, generator=g, device="cuda").half().t()
+    x = flat[1:].view(300, 64)
+    ref = x.double() @ w.double().t()
+    check(_ops.matmul_nt(x, w), ref, x.double().abs() @ w.double().abs().t(), 64)
+
+
+def make_layer(N, K, bits, gs, act, seed, packed=True, fractional=False):
+    from distributed_gptq_amd.models import QuantizedLinear
+    rng = np.random.default_rng(seed)
+    ng = -(-K // gs)
+    codes = torch.from_numpy(rng.integers(0, 2 ** bits, (N, K)).astype(np.uint8)).cuda()
+    scales = torch.from_numpy(rng.uniform(1e-3, 1e-2, (N, ng))).half().cuda()
+    zeros = rng.integers(0, 2 ** bits, (N, ng)).astype(np.float64)
+    if fractional:
+        zeros[N // 2, ng - 1] += 0.375  # one zero point off the integers
+    zeros = torch.from_numpy(zeros).half().cuda()
+    gi = torch.arange(K, dtype=torch.int32, device="cuda") // gs
+    if act:
+        gi = gi[torch.from_numpy(rng.permutation(K)).cuda()]
+    q = QuantizedLinear(bits, gs, K, N, bias=False, packed=packed).cuda()
+    q.pack_weights(codes, scales, zeros, gi)
+    W = (codes.double() - zeros.double()[:, gi.long()]) * scales.double()[:, gi.long()]
+    return q, W
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,K,bits,gs,act,packed,fractional", [
+    (64, 32, 4, 32, False, True, False),      # the smallest
+    (192, 160, 3, 32, True, True, False),     # columns past a 128-column block
+    (576, 1056, 2, 96, False, True, False),
+    (128, 288, 8, 288, False, True, False),   # three planes
+    (128, 288, 8, 96, True, False, False),    # one code per byte
+    (320, 416, 4, 32, True, True, True),      # a fractional zero: three planes
+])
+def test_input_gradient_planes(N, K, bits, gs, act, packed, fractional, dtype):
+    from distributed_gptq_amd import _ops
+    q, W = make_layer(N, K, bits, gs, act, N + K + bits, packed, fractional)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    perm = q.perm if q.perm.numel() else None
+    for M in (1, 130, 300):
+        go = (torch.randn(M, N, generator=g, device="cuda") * 1e-2).to(dtype)
+        gx = _ops.linear_grad_input(go, q.qweight, bits if packed else 0, q.scales, q.zeros, K, gs, perm)
+        # (the fp32 weight rounds (q - z) s once, the planes hold that value)
+        check(gx, go.double() @ W, go.double().abs() @ W.abs(), 6 * N)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_input_gradient_of_infinities(dtype):
+    """An infinite or NaN gradient gives what the unsplit product gives: the
+    weights' zero low planes are no terms of the sum."""
+    from distributed_gptq_amd import _ops
+    q, W = make_layer(128, 256, 4, 64, False, 5)
+    go = torch.randn(70, 128, device="cuda").to(dtype)
+    go[3, 17] = float("inf")
+    go[40, 5] = float("nan")
+    go[66, 100] = -float("inf")
+    gx = _ops.linear_grad_input(go, q.qweight, 4, q.scales, q.zeros, 256, 64)
+    ref = (go.float() @ W.float()).to(dtype)
+    assert torch.equal(torch.isnan(gx), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert inf.any() and torch.equal(gx[inf], ref[inf]) and torch.equal(torch.isinf(gx), inf)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("act", [False, True])
+def test_operator_routes(dtype, act):
+    """Forward on the dense kernel, backward on the planes, through the
+    operator, and the routes a differentiated or batched gradient takes."""
+    from distributed_gptq_amd.models import layers
+    N, K, M = 4096, 128, 1536
+    assert layers._dense_forward(M, N, K) and layers._planes_backward(M, 256, 4096, 4, dtype, None)
+    q, W = make_layer(N, K, 4, 64, act, 9)
+    x = torch.randn(M, K, device="cuda").to(dtype)
+    with torch.no_grad():
+        y = q(x)
+    Wr = W.to(dtype).double()
+    check(y, x.double() @ Wr.t(), x.double().abs() @ Wr.abs().t(), K)
+    q, W = make_layer(256, 4096, 4, 64, act, 10)
+    x = torch.randn(M, 4096, device="cuda").to(dtype).requires_grad_(True)
+    go = (torch.randn(M, 256, device="cuda") * 1e-2).to(dtype)
+    y = q(x)
+    gx, = torch.autograd.grad(y, x, go, retain_graph=True)
+    check(gx, go.double() @ W, go.double().abs() @ W.abs(), 6 * 256)
+    # the gradient of the gradient: gx is linear in go
+    gr = go.clone().requires_grad_(True)
+    gx2, = torch.autograd.grad(y, x, gr, create_graph=True, retain_graph=True)
+    gg, = torch.autograd.grad(gx2.float().sum(), gr)
+    assert torch.isfinite(gg).all() and gg.shape == gr.shape
+    both, = torch.autograd.grad(y, x, torch.stack([go, go]), is_grads_batched=True)
+    assert both.shape == (2, M, 4096)
 
 
 @pytest.mark.parametrize("bits", [2, 3, 4, 8])
