@@ -373,6 +373,9 @@ void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ld
   int s, tile, I, J;
   split_tile<2>(blockIdx.x, S, ntiles, s, tile);
   band_coords(tile, static_cast<int>(cdiv(static_cast<int64_t>(K), kTile)), I, J);
+  // (wave-uniform, but computed through the vector unit's square root)
+  I = __builtin_amdgcn_readfirstlane(I);
+  J = __builtin_amdgcn_readfirstlane(J);
   const bool diag = (I == J);
   const int64_t tb = static_cast<int64_t>(uniform_u64(static_cast<uint64_t>(static_cast<int64_t>(s) * tok_per_split)));
   const int64_t te = static_cast<int64_t>(uniform_u64(static_cast<uint64_t>(min(n, tb + tok_per_split))));
@@ -407,8 +410,9 @@ void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ld
   };
   auto stage_src = [&](int64_t t0) {
     const int rem = static_cast<int>(te - t0);
-    const int rows = rem <= 0 ? 0 : rem < kBK ? rem : kBK;
-    const uint32_t nrec = static_cast<uint32_t>(rows * rowb);
+    // (the clamp becomes a vector median: back to a scalar)
+    const int rows = __builtin_amdgcn_readfirstlane(rem <= 0 ? 0 : rem < kBK ? rem : kBK);
+    const uint32_t nrec = static_cast<uint32_t>(rows) * static_cast<uint32_t>(rowb);
     StageSrc ss;
 #pragma unroll
     for (int op = 0; op < 2; ++op) {
@@ -482,6 +486,7 @@ void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ld
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // MFMA
       if constexpr (m < 8) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);      // LDS reads
       if constexpr (step_copy(m) >= 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // copy
+      __builtin_amdgcn_sched_group_barrier(0x004, 2, 0);                          // scalar work
     });
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -489,12 +494,17 @@ void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ld
   // stage at t0 out of buffer B, its step-0 fragments already in set 0.  The
   // tail after the barrier runs also after the split's last stage: its
   // copies then have zero records and its reads go unused.
+  StageSrc ahead2;
   auto stage = [&](int64_t t0, auto bsel) {
     constexpr int B = decltype(bsel)::value;
     using Bn = std::integral_constant<int, (B + 1) % 3>;
     using Bp = std::integral_constant<int, (B + 2) % 3>;
-    const StageSrc ahead2 = stage_src(t0 + 2 * kBK);
+    // the scalar work for the copies after the barrier, done (and pinned)
+    // before it, under MFMAs: after it, the MFMA pipe would wait for it
+    StageSrc ahead3 = stage_src(t0 + 3 * kBK);
+    uint64_t b0 = reinterpret_cast<uint64_t>(ahead3.base[0]), b1 = reinterpret_cast<uint64_t>(ahead3.base[1]);
     step(I0{}, bsel, I1{}, I1{}, ahead2, Bp{}, std::integral_constant<int, 4>{});
+    asm volatile("" : "+s"(b0), "+s"(b1), "+s"(ahead3.nrec[0]), "+s"(ahead3.nrec[1]));
     step(I1{}, bsel, I2{}, I2{}, ahead2, Bp{}, std::integral_constant<int, 8>{});
     sfor<0, 8>([&](auto mc) { mfma(I2{}, mc); });
     __builtin_amdgcn_sched_barrier(0);
@@ -502,7 +512,8 @@ void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ld
     wait_lgkm<0>();
     bare_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    const StageSrc ahead3 = stage_src(t0 + 3 * kBK);
+    ahead3.base[0] = reinterpret_cast<const uint16_t*>(b0);
+    ahead3.base[1] = reinterpret_cast<const uint16_t*>(b1);
     sfor<8, 16>([&](auto mc) {
       constexpr int m = decltype(mc)::value;
       mfma(I2{}, mc);
@@ -516,6 +527,7 @@ void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ld
       if constexpr (tail_copy(m) >= 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
     });
     __builtin_amdgcn_sched_barrier(0);
+    ahead2 = ahead3;
   };
 
   if (tb < te) {
@@ -532,6 +544,7 @@ void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ld
     // three stages per trip, one per buffer; stages past the split's end
     // multiply zeros, which leaves the sums unchanged (+0 added to a sum that
     // starts at +0)
+    ahead2 = s2;
     for (int64_t t0 = tb; t0 < te; t0 += 3 * kBK) {
       stage(t0, I0{});
       stage(t0 + kBK, I1{});
