@@ -6,12 +6,15 @@
 //     grid, each wave owning a 128 x 128 block = 4 x 4 MFMA 32x32 blocks (256
 //     fp32 accumulators per lane, in AGPRs).
 //   * The tokens are cut into S contiguous splits (choose_splits: at most
-//     16384 tokens each).  Workgroup b works on the (split, tile) pair that
-//     split_tile maps it to: split-major, tiles in band order, each round of
-//     256 workgroups permuted so that every XCD runs 32 neighbouring tiles.
+//     16384 tokens each).  hessian_gram16 cuts the tiles past its last full
+//     round of workgroups finer (hessian_plan).  Workgroup b works on the
+//     (split, tile) pair that split_tile maps it to: split-major, tiles in
+//     band order, each round of 256 workgroups permuted so that every XCD runs
+//     neighbouring tiles.
 //   * Each (split, tile) writes an fp32 partial tile to the workspace; a
 //     reduce kernel adds the S partials in fixed order (deterministic) to the
-//     lower triangle of H and mirrors them to the upper triangle.
+//     lower triangle of H and mirrors them to the upper triangle.  A tile of
+//     one split is added to H by hessian_gram16 itself.
 //
 // Operands.  The Gram matrix needs, per lane, 8 consecutive tokens of one
 // feature (the k-run of v_mfma_f32_32x32x16_{bf16,f16}); X is stored token-
@@ -78,32 +81,12 @@ __host__ __device__ __forceinline__ void band_coords(int t, int T, int& I, int& 
 // (32 banks) or 16 lanes (64 banks).
 __device__ __forceinline__ int swz(int f) { return f ^ (((f >> 4) ^ ((f >> 1) & 4)) & 7); }
 
-// Workgroup b -> (split, tile).  Workgroups are dispatched round-robin over
-// the 8 XCDs, so XCD x runs b = x, x + 8, ...; with S a multiple of 8 it
-// walks every tile of split x, then of split x + 8, ...: the workgroups
-// resident on one XCD at a time share one token range and neighbouring
-// feature blocks, which its L2 then serves.
-template <int kMap = 0>
+// Workgroup b -> (split, tile) of S splits of every tile.  Workgroups are
+// dispatched round-robin over the 8 XCDs, so XCD x runs b = x, x + 8, ...;
+// with S a multiple of 8 it walks every tile of split x, then of split x + 8,
+// ...: the workgroups resident on one XCD at a time share one token range and
+// neighbouring feature blocks, which its L2 then serves.
 __host__ __device__ __forceinline__ void split_tile(int b, int S, int ntiles, int& s, int& tile) {
-  if (kMap == 1) {  // split-major: all XCDs on the same split
-    s = b / ntiles;
-    tile = b % ntiles;
-    return;
-  }
-  if (kMap == 2) {
-    // split-major over band-ordered tiles, with every round of 256
-    // workgroups (8 XCDs x 32 CUs) permuted so that XCD x runs 32 consecutive
-    // entries of that order: b = 8q + x -> entry 32 (8 (q / 32) + x) + q % 32.
-    // The last partial round keeps b itself.
-    int idx = b;
-    if (b < ((S * ntiles) & ~255)) {
-      const int x = b & 7, q = b >> 3;
-      idx = (((q >> 5) << 3) + x) * 32 + (q & 31);
-    }
-    s = idx / ntiles;
-    tile = idx % ntiles;
-    return;
-  }
   if (S % 8 == 0) {
     const int x = b & 7, q = b >> 3;
     s = x + 8 * (q / ntiles);
@@ -112,6 +95,30 @@ __host__ __device__ __forceinline__ void split_tile(int b, int S, int ntiles, in
     s = b % S;
     tile = b / S;
   }
+}
+
+// The splits of a launch of hessian_gram16 (plan::HessPlan): the first `whole`
+// tiles in s1 splits of per1 tokens, the others (the tail) in s2 of per2.
+struct HessSplit {
+  int s1, whole, s2;
+  int64_t per1, per2;
+};
+
+// Workgroup b of `grid` -> (split, tile), split-major over band-ordered tiles,
+// the first tiles' splits before the tail's, with every round of 256
+// workgroups (8 XCDs x 32 CUs; the last one what is left) permuted so that
+// XCD x runs consecutive entries of that order.  True for a tail tile.
+__device__ __forceinline__ bool split_tile(int b, int grid, const HessSplit& sp, int ntiles, int& s, int& tile) {
+  const int r0 = b & ~255, x = b & 7, q = (b & 255) >> 3;
+  const int w = grid - r0 < 256 ? grid - r0 : 256;
+  int idx = r0 + x * (w >> 3) + (x < (w & 7) ? x : (w & 7)) + q;
+  const int first = sp.s1 * sp.whole;
+  const bool tail = idx >= first;
+  if (tail) idx -= first;
+  const int count = tail ? ntiles - sp.whole : sp.whole;
+  s = idx / count;
+  tile = idx - s * count + (tail ? sp.whole : 0);
+  return tail;
 }
 
 // ------------------------------------------------------- 16-bit inputs ----
@@ -358,6 +365,25 @@ __device__ __forceinline__ uint8_t* hslab(int op) {
   return B == 0 ? &g_hslab0[op][0] : B == 1 ? &g_hslab1[op][0] : &g_hslab2[op][0];
 }
 
+// fp32 elements of a tile of H through a buffer descriptor: lane offset v,
+// wave-uniform offset s, in bytes; a negative v is past every record (loads
+// read zeros, stores do nothing)
+struct TileRsrc {
+  __amdgpu_buffer_rsrc_t rs;
+  __device__ __forceinline__ explicit TileRsrc(float* p)
+      : rs(__builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<float*>(uniform_u64(reinterpret_cast<uint64_t>(p))),
+                                             static_cast<short>(0), INT32_MAX, 0x00020000)) {}
+  __device__ __forceinline__ f32x4 load4(int v, int s) const {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, v, s, 0));
+  }
+  __device__ __forceinline__ void store4(const f32x4& x, int v, int s) const {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), rs, v, s, 0);
+  }
+  __device__ __forceinline__ void store1(float x, int v, int s) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), rs, v, s, 0);
+  }
+};
+
 // copy slots: after which MFMA m of a step the step's j-th copy goes (-1:
 // none), and after which MFMA m (8..15) of the last step's tail
 constexpr int step_copy(int m) { return m % 4 == 1 ? m / 4 : -1; }
@@ -365,13 +391,14 @@ constexpr int tail_copy(int m) { return m % 2 == 1 ? (m - 9) / 2 : -1; }
 
 template <bool kBF16>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ldx, int S, int64_t tok_per_split,
-                    int ntiles, float* __restrict__ partial) {
+void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ldx, HessSplit sp, int ntiles,
+                    float* __restrict__ partial, float* __restrict__ H) {
   constexpr int kBK = kDmaBK;
   constexpr int kPerWave = kBK / 4;  // 12 copies of 1 KB per wave and stage: 6 of each operand
 
   int s, tile, I, J;
-  split_tile<2>(blockIdx.x, S, ntiles, s, tile);
+  const bool tail = split_tile(blockIdx.x, gridDim.x, sp, ntiles, s, tile);
+  const int64_t tok_per_split = tail ? sp.per2 : sp.per1;
   band_coords(tile, static_cast<int>(cdiv(static_cast<int64_t>(K), kTile)), I, J);
   // (wave-uniform, but computed through the vector unit's square root)
   I = __builtin_amdgcn_readfirstlane(I);
@@ -464,7 +491,8 @@ void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ld
   };
   auto mfma = [&](auto ssel, auto msel) {
     constexpr int St = decltype(ssel)::value, m = decltype(msel)::value;
-    mfma32_asm<kBF16>(acc[m >> 2][m & 3], fr[St][m >> 2], fr[St][4 + (m & 3)]);
+    // (J's features first: a lane's accumulators then run along a row of the tile)
+    mfma32_asm<kBF16>(acc[m >> 2][m & 3], fr[St][4 + (m & 3)], fr[St][m >> 2]);
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
@@ -555,21 +583,91 @@ void hessian_gram16(const uint16_t* __restrict__ X, int64_t n, int K, int64_t ld
     mfma_settle();  // the accumulators are read below
   }
 
-  // 32x32 accumulator layout: lane l, register v -> row 8*(v/4) + 4*(l/32) + v%4, col l%32
+  // lane l, register v of block (i, j): row 32i + l % 32 of the tile, column
+  // 32j + 8 (v / 4) + 4 (l / 32) + v % 4
   if (wave_idle) return;
-  // partials are stored in the row-major triangle order the reduce reads
-  const int slot = I * (I + 1) / 2 + J;
-  float* out = partial + (static_cast<int64_t>(s) * ntiles + slot) * (kTile * kTile);
+  const int row0 = wm + (lane & 31), col0 = wn + 4 * (lane >> 5);
+  if (sp.s1 == 1 && !tail) {
+    // a tile of one split: added to H here and mirrored (the sums reduce
+    // would write; its pass over partial tiles took a sixth of a 16384-token
+    // call at K = 14336)
+    // Through buffer descriptors at the tile and at its mirror image: 32-bit
+    // lane offsets and scalar row offsets keep the addresses out of the vector
+    // registers.  Rows and columns past K get an offset past every record (the
+    // columns in groups of 8, inside or outside as a whole: K % 8 == 0 here).
+    // A block on the diagonal holds both triangles, equal bit for bit (the
+    // same products in the same order), and needs no mirroring.
+    const TileRsrc lower(H + static_cast<int64_t>(I) * kTile * K + J * kTile);
+    const TileRsrc upper(H + static_cast<int64_t>(J) * kTile * K + I * kTile);
+    const int rowsK = 4 * K;  // bytes of a row
+    const int vlow = row0 * rowsK + 4 * col0, vup = col0 * rowsK + 4 * row0;
+    const int left_r = K - I * kTile - row0, left_c = K - J * kTile - wn;
+    const bool mirror = !(diag && wm == wn);
+    f32x4 hv[2][4][4];  // H of two rows of blocks: the next one's loads are in flight
+    auto load = [&](auto isel) {
+      constexpr int i = decltype(isel)::value;
+      const int v = 32 * i < left_r ? vlow : INT32_MIN;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int c = 32 * j + 8 * q;
+          hv[i & 1][j][q] = lower.load4(c < left_c ? v + 4 * c : INT32_MIN, 32 * i * rowsK);
+        }
+    };
+    load(I0{});
+    sfor<0, 4>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (i < 3) load(std::integral_constant<int, i + 1>{});
+      __builtin_amdgcn_sched_barrier(0);
+      const bool rin = 32 * i < left_r;
+      const int vl = rin ? vlow : INT32_MIN, vu = rin && mirror ? vup : INT32_MIN;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        // (stays in AGPRs up to here: copied out earlier, all blocks spilled)
+        asm volatile("" : "+a"(acc[i][j]));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int c = 32 * j + 8 * q;
+          const bool cin = c < left_c;
+          f32x4 h = hv[i & 1][j][q];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) h[e] = acc[i][j][4 * q + e] + h[e];
+          lower.store4(h, cin ? vl + 4 * c : INT32_MIN, 32 * i * rowsK);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) upper.store1(h[e], cin ? vu + 128 * i : INT32_MIN, (c + e) * rowsK);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+    return;
+  }
+  // partial tiles: those of the first tiles split by split, then the tail's
+  const int64_t first = sp.s1 == 1 ? 0 : static_cast<int64_t>(sp.s1) * sp.whole;
+  const int64_t slot = tail ? first + static_cast<int64_t>(s) * (ntiles - sp.whole) + (tile - sp.whole)
+                            : static_cast<int64_t>(s) * sp.whole + tile;
+  // in the accumulators' order, [wave][i][j][q][lane] of four columns each, so
+  // that a store is 1 KB of consecutive bytes (in the tile's rows it was 32 of
+  // 32 bytes); partial_quad is the reduce's way back
+  f32x4* out = reinterpret_cast<f32x4*>(partial + slot * (kTile * kTile)) + wave * 4096 + lane;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      asm volatile("" : "+a"(acc[i][j]));
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = wm + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        const int col = wn + j * 32 + (lane & 31);
-        out[row * kTile + col] = acc[i][j][v];
-      }
+      for (int q = 0; q < 4; ++q)
+        out[((i * 4 + j) * 4 + q) * 64] =
+            f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+    }
+}
+
+// Index of the four values at (row, col .. col + 3), col % 4 == 0, of a
+// hessian_gram16 partial tile.
+__device__ __forceinline__ int partial_quad(int row, int col) {
+  const int wave = (row >> 7) * 2 + (col >> 7), i = (row >> 5) & 3, j = (col >> 5) & 3, q = (col >> 3) & 3;
+  return wave * 4096 + ((i * 4 + j) * 4 + q) * 64 + (row & 31) + 32 * ((col >> 2) & 1);
 }
 
 // --------------------------------------------------------- fp32 inputs ----
@@ -695,22 +793,33 @@ void hessian_tile32(const float* __restrict__ X, int64_t n, int K, int64_t ldx, 
 // One workgroup per 32 x 32 sub-block of a lower tile.  H[gi][gj] (gi >= gj
 // within diagonal sub-blocks) += sum_s partial[s]; the sum is mirrored to
 // H[gj][gi] through an LDS transpose so H stays exactly symmetric.
+template <bool kBand>
 __global__ __launch_bounds__(256) void hessian_reduce(float* __restrict__ H, int K, const float* __restrict__ partial,
-                                                      int S, int ntiles) {
+                                                      HessSplit sp, int ntiles) {
   __shared__ float t[32][33];
-  const int tile = blockIdx.x >> 6;
+  // the tiles that have partials: all of them, or those after the `whole`
+  // ones that the tile kernel added to H itself
+  const int tile = (blockIdx.x >> 6) + (sp.s1 == 1 && kBand ? sp.whole : 0);
+  const bool tail = tile >= sp.whole;
+  const int S = tail ? sp.s2 : sp.s1;
+  const int64_t count = tail ? ntiles - sp.whole : sp.whole;  // tiles of this kind: the stride of a split
+  const int64_t first = tail ? (sp.s1 == 1 && kBand ? 0 : static_cast<int64_t>(sp.s1) * sp.whole) : 0;
   const int sb = blockIdx.x & 63;
   const int sr = sb >> 3, sc = sb & 7;
   int I, J;
-  tile_coords(tile, I, J);
+  if (kBand)
+    band_coords(tile, static_cast<int>(cdiv(static_cast<int64_t>(K), kTile)), I, J);
+  else
+    tile_coords(tile, I, J);
   if (I == J && sc > sr) return;
   const bool diag_sb = (I == J) && (sr == sc);
   const int tid = threadIdx.x;
   const int row = tid >> 3;
   const int col0 = (tid & 7) * 4;
   const int64_t gi = static_cast<int64_t>(I) * kTile + sr * 32 + row;
-  const int64_t tstride = static_cast<int64_t>(ntiles) * kTile * kTile;
-  const float* p = partial + static_cast<int64_t>(tile) * kTile * kTile + (sr * 32 + row) * kTile + sc * 32 + col0;
+  const int64_t tstride = count * kTile * kTile;
+  const float* p = partial + (first + (tail ? tile - sp.whole : tile)) * kTile * kTile +
+                   (kBand ? 4 * partial_quad(sr * 32 + row, sc * 32 + col0) : (sr * 32 + row) * kTile + sc * 32 + col0);
   // partials summed in split order; up to eight loads are issued before
   // their adds (the last < 8 as well: one at a time, each waited for, they
   // were a chain of round trips with 4 splits)
@@ -775,8 +884,8 @@ namespace gptq {
 namespace {
 
 // H += X^T X for one run of tokens with S splits, partials in `part`
-int accumulate_run(float* H, const void* X, int64_t n, int64_t K, int64_t ldx, int dtype, int S, float* part,
-                   hipStream_t st) {
+int accumulate_run(float* H, const void* X, int64_t n, int64_t K, int64_t ldx, int dtype, int S, bool fits,
+                   float* part, hipStream_t st) {
   const int64_t T = cdiv(K, kTile);
   const int ntiles = static_cast<int>(T * (T + 1) / 2);
   const int64_t per = cdiv(cdiv(n, S), 32) * 32;
@@ -795,21 +904,35 @@ int accumulate_run(float* H, const void* X, int64_t n, int64_t K, int64_t ldx, i
     const uint16_t* x = static_cast<const uint16_t*>(X);
     // aligned rows: LDS-DMA kernel, 4 waves of 128 x 128, split-major band
     // order; otherwise the register-staged kernel with element loads
+    if (vec) {
+      plan::HessPlan p{S, ntiles, 1};
+      if (fits) p = plan::hessian_plan(n, ntiles, S);
+      auto tokens = [&](int splits) { return cdiv(cdiv(n, splits), 32) * 32; };
+      const HessSplit sp{p.s1, static_cast<int>(p.whole), p.s2, tokens(p.s1), tokens(p.s2)};
+      const int64_t units = static_cast<int64_t>(p.s1) * p.whole + static_cast<int64_t>(p.s2) * (ntiles - p.whole);
+      const dim3 g(static_cast<unsigned>(units));
+      if (dtype == GPTQ_BF16)
+        hipLaunchKernelGGL(hessian_gram16<true>, g, dim3(256), 0, st, x, n, (int)K, ldx, sp, ntiles, part, H);
+      else
+        hipLaunchKernelGGL(hessian_gram16<false>, g, dim3(256), 0, st, x, n, (int)K, ldx, sp, ntiles, part, H);
+      const int rc = check_launch("hessian_gram");
+      const int64_t left = p.s1 == 1 ? ntiles - p.whole : ntiles;  // tiles with partials
+      if (rc || left == 0) return rc;
+      hipLaunchKernelGGL(hessian_reduce<true>, dim3(static_cast<unsigned>(left) * 64), dim3(256), 0, st, H, (int)K, part,
+                         sp, ntiles);
+      return check_launch("hessian_reduce");
+    }
     if (dtype == GPTQ_BF16) {
-      if (vec)
-        hipLaunchKernelGGL((hessian_gram16<true>), grid, dim3(256), 0, st, x, n, (int)K, ldx, S, per, ntiles, part);
-      else
-        hipLaunchKernelGGL((hessian_tile16<true, false>), grid, dim3(kThreads16), 0, st, x, n, (int)K, ldx, S, per, ntiles, part);
+      hipLaunchKernelGGL((hessian_tile16<true, false>), grid, dim3(kThreads16), 0, st, x, n, (int)K, ldx, S, per, ntiles, part);
     } else {
-      if (vec)
-        hipLaunchKernelGGL((hessian_gram16<false>), grid, dim3(256), 0, st, x, n, (int)K, ldx, S, per, ntiles, part);
-      else
-        hipLaunchKernelGGL((hessian_tile16<false, false>), grid, dim3(kThreads16), 0, st, x, n, (int)K, ldx, S, per, ntiles, part);
+      hipLaunchKernelGGL((hessian_tile16<false, false>), grid, dim3(kThreads16), 0, st, x, n, (int)K, ldx, S, per, ntiles, part);
     }
   }
-  int rc = check_launch("hessian_tile");
+  const int rc = check_launch("hessian_tile");
   if (rc) return rc;
-  hipLaunchKernelGGL(hessian_reduce, dim3(static_cast<unsigned>(ntiles) * 64), dim3(256), 0, st, H, (int)K, part, S, ntiles);
+  const HessSplit sp{S, ntiles, 1, per, per};
+  hipLaunchKernelGGL(hessian_reduce<false>, dim3(static_cast<unsigned>(ntiles) * 64), dim3(256), 0, st, H, (int)K, part,
+                     sp, ntiles);
   return check_launch("hessian_reduce");
 }
 
@@ -833,7 +956,7 @@ extern "C" int gptq_hessian_accumulate(float* H, const void* X, int64_t n, int64
   hipStream_t st = as_hip(stream);
   const int S = plan::choose_splits(n, ntiles);
   if (static_cast<size_t>(S) * split_bytes <= workspace_bytes)
-    return accumulate_run(H, X, n, K, ldx, dtype, S, part, st);
+    return accumulate_run(H, X, n, K, ldx, dtype, S, true, part, st);
   // a smaller workspace: consecutive runs of tokens, each with as many splits
   // as the workspace holds, added to H one after the other (fixed order)
   const int64_t cap = static_cast<int64_t>(workspace_bytes / split_bytes);
@@ -842,7 +965,7 @@ extern "C" int gptq_hessian_accumulate(float* H, const void* X, int64_t n, int64
   for (int64_t t0 = 0; t0 < n; t0 += run) {
     const int64_t m = std::min<int64_t>(run, n - t0);
     const int Sm = static_cast<int>(std::min<int64_t>(plan::choose_splits(m, ntiles), cap));
-    const int rc = accumulate_run(H, static_cast<const char*>(X) + t0 * ldx * esz, m, K, ldx, dtype, Sm, part, st);
+    const int rc = accumulate_run(H, static_cast<const char*>(X) + t0 * ldx * esz, m, K, ldx, dtype, Sm, false, part, st);
     if (rc) return rc;
   }
   return GPTQ_OK;

@@ -40,6 +40,18 @@ int64_t hessian_tiles(int64_t K);
 size_t hessian_split_bytes(int64_t K);
 // token splits of one launch over n tokens (1..64)
 int choose_splits(int64_t n, int64_t ntiles);
+// How one launch of the 16-bit tile kernel cuts n tokens: the first `whole` of
+// the tiles (in the kernel's order) into s1 splits each, the others into s2.
+// With s1 == 1 the first tiles are added to H by the tile kernel itself and
+// have no partial tiles.
+struct HessPlan {
+  int s1;
+  int64_t whole;
+  int s2;
+};
+// `splits`: what choose_splits gives; the plan's partial tiles fit in
+// splits * ntiles
+HessPlan hessian_plan(int64_t n, int64_t ntiles, int splits);
 // tokens per run when the workspace holds only `cap` splits' partial tiles
 // (fewer than choose_splits wants): runs are added to H one after the other
 int64_t hessian_run_tokens(int64_t ntiles, int64_t cap);
