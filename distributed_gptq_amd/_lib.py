@@ -17,6 +17,7 @@ import torch  # noqa: F401  (must precede the library load, see module doc)
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libgptq_hip.so")
+TORCH_OPS_PATH = os.path.join(HERE, "libgptq_torch.so")  # the native torch operator (csrc/torch_ops.cc)
 
 # status codes (gptq_status)
 OK, ERR_ARG, ERR_SHAPE, ERR_DTYPE, ERR_WORKSPACE, ERR_LAUNCH, ERR_DEVICE = range(7)
@@ -99,6 +100,21 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
                 fn.argtypes = args
             _handle = h
         return _handle
+
+
+_torch_ops = False
+
+
+def load_torch_ops(path: str = TORCH_OPS_PATH):
+    """Register the native torch operators (once)."""
+    global _torch_ops
+    load()
+    with _lock:
+        if not _torch_ops:
+            if not os.path.exists(path):
+                raise ImportError(f"{path} is not built: run `python -m distributed_gptq_amd.build`")
+            torch.ops.load_library(path)
+            _torch_ops = True
 
 
 def lib() -> ctypes.CDLL:

@@ -4,7 +4,9 @@
 
 Every ``.hip``/``.cpp`` under ``csrc/`` is compiled with hipcc to an object
 under ``csrc/_build/`` (in parallel) and linked into
-``distributed_gptq_amd/libgptq_hip.so``.
+``distributed_gptq_amd/libgptq_hip.so``; ``csrc/torch_ops.cc``, the native
+torch operator over it, is compiled with g++ against torch's headers into
+``distributed_gptq_amd/libgptq_torch.so``.
 """
 from __future__ import annotations
 
@@ -16,6 +18,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libgptq_hip.so")
+TORCH_OUT = os.path.join(HERE, "libgptq_torch.so")
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -47,6 +50,24 @@ def _compile(src, objdir, extra):
     return obj, r.stderr
 
 
+def build_torch_ops():
+    """libgptq_torch.so (host code only; needs libgptq_hip.so to link)."""
+    import torch
+    base = os.path.dirname(torch.__file__)
+    tmp = TORCH_OUT + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I", os.path.join(os.path.dirname(HERE), "include"), "-isystem", os.path.join(base, "include"),
+           "-isystem", "/opt/rocm/include", os.path.join(CSRC, "torch_ops.cc"), "-o", tmp, "-L", HERE,
+           "-l:libgptq_hip.so", "-L", os.path.join(base, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on torch_ops.cc:\n{r.stderr}")
+    os.replace(tmp, TORCH_OUT)
+    return TORCH_OUT
+
+
 def build(verbose=False, extra=()):
     objdir = os.path.join(CSRC, "_build")
     os.makedirs(objdir, exist_ok=True)
@@ -64,6 +85,7 @@ def build(verbose=False, extra=()):
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr}")
     os.replace(tmp, OUT)
+    build_torch_ops()
     return OUT
 
 
