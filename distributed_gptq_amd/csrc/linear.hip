@@ -1079,7 +1079,9 @@ __device__ __forceinline__ void stage_sz(const LinArgs& a, int64_t n0, float2* s
   const char* sb = static_cast<const char*>(a.scales) + n0 * a.ngroups * esz;
   const char* zb = static_cast<const char*>(a.zeros) + n0 * a.ngroups * esz;
   if (((reinterpret_cast<uintptr_t>(sb) | reinterpret_cast<uintptr_t>(zb)) & 15u) == 0) {
-    const uint32_t bytes = static_cast<uint32_t>(std::min<int64_t>(NT, a.N - n0) * ng * esz);
+    // (whole words: a last half alone in its word would be out of range; the
+    // word lies inside the allocation, as in elem_word)
+    const uint32_t bytes = (static_cast<uint32_t>(std::min<int64_t>(NT, a.N - n0) * ng * esz) + 3u) & ~3u;
     const __amdgpu_buffer_rsrc_t srs = make_rsrc(sb, bytes), zrs = make_rsrc(zb, bytes);
     const int epv = 16 / esz;
     const int nvec = static_cast<int>(cdiv(tot, epv));
@@ -1096,7 +1098,7 @@ __device__ __forceinline__ void stage_sz(const LinArgs& a, int64_t n0, float2* s
       };
       if (esz == 4) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) put(__builtin_bit_cast(float, sv[j]), __builtin_bit_cast(float, zv[j]));
+        for (int j = 0; j < 4; ++j) put(__uint_as_float(sv[j]), __uint_as_float(zv[j]));  // (a bit cast of sv[j] is sv[0])
       } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j)
