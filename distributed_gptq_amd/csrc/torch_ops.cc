@@ -30,12 +30,12 @@ at::Tensor linear_rows(const at::Tensor& x, const at::Tensor& qweight, const at:
                   zeros.device() == x.device() && (!bias || bias->device() == x.device()) &&
                   (!perm || perm->device() == x.device()),
               "gptq::linear_rows: expected GPU tensors on one device");
-  TORCH_CHECK_VALUE(K > 0 && x.dim() > 0 && qweight.dim() == 2 && scales.dim() == 2 &&
+  TORCH_CHECK_VALUE(K > 0 && x.dim() > 0 && x.size(-1) == K && qweight.dim() == 2 && scales.dim() == 2 &&
                         zeros.sizes() == scales.sizes() && scales.size(0) == qweight.size(0) &&
                         qweight.scalar_type() == at::kByte && qweight.is_contiguous() &&
                         qweight.size(1) == (bits == 0 ? K : (K * bits + 7) / 8) &&
                         (!bias || bias->numel() == qweight.size(0)),
-                    "gptq::linear_rows: the weight's shapes do not match in_features = ", K);
+                    "gptq::linear_rows: the shapes of x and the weight do not match in_features = ", K);
   const c10::DeviceGuard guard(x.device());
   const int64_t N = qweight.size(0);
   const at::Tensor x2 = x.reshape({-1, K}).contiguous();

@@ -308,7 +308,7 @@ def _apply_linear(x, qweight, scales, zeros, g_idx, bias, perm):
     that refuses is left to gptq::linear, which raises or computes it."""
     if perm is not None and not perm.numel():
         perm = None
-    if type(x) is torch.Tensor and x.is_cuda and not (
+    if type(x) is torch.Tensor and x.is_cuda and not torch.compiler.is_compiling() and not (
             (torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad)))
             or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
             or torch._C._functorch.peek_interpreter_stack() is not None or torch.jit.is_tracing()):

@@ -76,6 +76,9 @@ def test_calls_left_to_the_operator():
             q(x.double())
         with pytest.raises(ValueError):
             q(x[:0])
+        for shape in ((8, 1024), (8, 256), (1024,)):  # whole rows of K, but not K wide
+            with pytest.raises(RuntimeError):
+                q(torch.zeros(shape, device="cuda").half())
         q.qweight.data = q.qweight[:, :-1].contiguous()
         with pytest.raises(ValueError):
             q(x)
