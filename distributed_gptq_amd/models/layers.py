@@ -102,10 +102,11 @@ def _group_layout(g_idx: torch.Tensor, K: int, ngroups: int, perm: Optional[torc
 
 
 # Rows of x from which the weights are dequantised once (to x's dtype) and
-# multiplied by the library GEMM instead of the fused kernels, which decode
+# multiplied as a dense product instead of the fused kernels, which decode
 # every weight once per 128 rows.  Measured on MI355X (4-bit, fp16/bf16, the
-# Llama-3-8B and 13B layer shapes): at 384 rows the two are even or the GEMM
-# wins, at 512 it wins everywhere, at 16384 rows by 3.4-3.7x.
+# Llama-3-8B and 13B layer shapes, the product in the library): at 384 rows
+# the two are even or the product wins, at 512 it wins everywhere, at 16384
+# rows by 3.4-3.7x.
 DEQUANT_GEMM_ROWS = 384
 
 
@@ -219,7 +220,10 @@ def _linear_impl(x, qweight, scales, zeros, g_idx, bias, perm=None):
         # x's dtype (a 16-bit product may otherwise reduce split-K partials in
         # 16 bits, torch's allow_*_reduced_precision_reduction default)
         x2 = x.reshape(-1, K)
-        if _dense_forward(rows, W.shape[0], K):
+        # (other biases keep the library's broadcast, conversion and errors)
+        plain_bias = bias is None or (bias.shape == W.shape[:1] and bias.device == x.device and
+                                      bias.dtype in (torch.float32, torch.float16, torch.bfloat16))
+        if plain_bias and _dense_forward(rows, W.shape[0], K):
             return _ops.matmul_nt(x2, W, bias).reshape(*x.shape[:-1], W.shape[0])
         if bias is None:
             y = torch.mm(x2, W.t(), out_dtype=torch.float32)

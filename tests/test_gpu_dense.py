@@ -144,6 +144,25 @@ def test_operator_routes(dtype, act):
     assert both.shape == (2, M, 4096)
 
 
+def test_biases_of_the_library_product():
+    """Biases that the dense kernel does not read as N values of its types
+    keep the library product: its broadcast, its conversion and its errors."""
+    from distributed_gptq_amd.models import layers
+    N, K, M = 4096, 128, 1536
+    assert layers._dense_forward(M, N, K)
+    q, W = make_layer(N, K, 4, 64, False, 11)
+    x = torch.randn(M, K, device="cuda").half()
+    args = (x, q.qweight, q.scales, q.zeros, q.g_idx)
+    Wr, b = W.half().double(), torch.randn(N, device="cuda", dtype=torch.float64)
+    ref, mag = x.double() @ Wr.t(), x.double().abs() @ Wr.abs().t()
+    for bias in (b, b[:1]):
+        # the bias itself is rounded to fp32 once
+        check(torch.ops.gptq.linear(*args, bias), ref + bias, mag + bias.abs(), K + 2)
+    for bias in (b[:-1].float(), b.float().cpu()):
+        with pytest.raises(RuntimeError):
+            torch.ops.gptq.linear(*args, bias)
+
+
 @pytest.mark.parametrize("bits", [2, 3, 4, 8])
 @pytest.mark.parametrize("N,K,gs", [(1, 32, 32), (5, 96, 32), (7, 2080, 64), (66, 4096, 4096)])
 def test_dequant_rows(N, K, gs, bits):
