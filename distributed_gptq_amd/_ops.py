@@ -97,7 +97,7 @@ def hessian_accumulate(H: torch.Tensor, X: torch.Tensor, workspace_cap: int | No
     ldx = X2.stride(0) if n > 1 else K
     lib = L.lib()
     cap = HESSIAN_WORKSPACE_CAP if workspace_cap is None else workspace_cap
-    nb = min(lib.gptq_hessian_workspace_size(n, K), max(lib.gptq_hessian_workspace_min(K), cap))
+    nb = min(lib.gptq_hessian_workspace_best(n, K), max(lib.gptq_hessian_workspace_min(K), cap))
     ws = workspace(nb, H.device)
     L.call("gptq_hessian_accumulate", _p(H), _p(X2), n, K, ldx, dtype_code(X2.dtype), _p(ws), nb,
            _stream(H.device))

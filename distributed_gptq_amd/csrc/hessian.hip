@@ -883,8 +883,9 @@ using namespace gptq;
 namespace gptq {
 namespace {
 
-// H += X^T X for one run of tokens with S splits, partials in `part`
-int accumulate_run(float* H, const void* X, int64_t n, int64_t K, int64_t ldx, int dtype, int S, bool fits,
+// H += X^T X for one run of tokens with S splits, partials in `part`; room: the
+// splits' partials that it holds (0: equal splits)
+int accumulate_run(float* H, const void* X, int64_t n, int64_t K, int64_t ldx, int dtype, int S, int room,
                    float* part, hipStream_t st) {
   const int64_t T = cdiv(K, kTile);
   const int ntiles = static_cast<int>(T * (T + 1) / 2);
@@ -906,7 +907,7 @@ int accumulate_run(float* H, const void* X, int64_t n, int64_t K, int64_t ldx, i
     // order; otherwise the register-staged kernel with element loads
     if (vec) {
       plan::HessPlan p{S, ntiles, 1};
-      if (fits) p = plan::hessian_plan(n, ntiles, S);
+      if (room) p = plan::hessian_plan(n, ntiles, S, room);
       auto tokens = [&](int splits) { return cdiv(cdiv(n, splits), 32) * 32; };
       const HessSplit sp{p.s1, static_cast<int>(p.whole), p.s2, tokens(p.s1), tokens(p.s2)};
       const int64_t units = static_cast<int64_t>(p.s1) * p.whole + static_cast<int64_t>(p.s2) * (ntiles - p.whole);
@@ -955,8 +956,10 @@ extern "C" int gptq_hessian_accumulate(float* H, const void* X, int64_t n, int64
   float* part = static_cast<float*>(workspace);
   hipStream_t st = as_hip(stream);
   const int S = plan::choose_splits(n, ntiles);
+  const int room = plan::hessian_room(ntiles, S);
+  const size_t room_bytes = static_cast<size_t>(room) * split_bytes;
   if (static_cast<size_t>(S) * split_bytes <= workspace_bytes)
-    return accumulate_run(H, X, n, K, ldx, dtype, S, true, part, st);
+    return accumulate_run(H, X, n, K, ldx, dtype, S, room_bytes <= workspace_bytes ? room : S, part, st);
   // a smaller workspace: consecutive runs of tokens, each with as many splits
   // as the workspace holds, added to H one after the other (fixed order)
   const int64_t cap = static_cast<int64_t>(workspace_bytes / split_bytes);
@@ -965,7 +968,7 @@ extern "C" int gptq_hessian_accumulate(float* H, const void* X, int64_t n, int64
   for (int64_t t0 = 0; t0 < n; t0 += run) {
     const int64_t m = std::min<int64_t>(run, n - t0);
     const int Sm = static_cast<int>(std::min<int64_t>(plan::choose_splits(m, ntiles), cap));
-    const int rc = accumulate_run(H, static_cast<const char*>(X) + t0 * ldx * esz, m, K, ldx, dtype, Sm, false, part, st);
+    const int rc = accumulate_run(H, static_cast<const char*>(X) + t0 * ldx * esz, m, K, ldx, dtype, Sm, 0, part, st);
     if (rc) return rc;
   }
   return GPTQ_OK;

@@ -53,50 +53,49 @@ int choose_splits(int64_t n, int64_t ntiles) {
 // 6.2 rounds, (16384, 4096) in 4 splits 544 workgroups = 2.1 rounds.  Here the
 // tiles past the last full round are cut finer, so that they share one short
 // round.  By the time of a round (23.6 ns a token, 5 us of start and drain)
-// and of a partial tile's way through memory (0.15 us), measured on MI355X;
-// the split counts stay within choose_splits' bounds on tokens per split
-// (10240 below 512 tiles, 16384 below 1024) and at three quarters of its
-// count (half of it, 2 splits at (16384, 4096), was 1% faster and a little
-// less exact); from 1024 tiles on it is its count.
+// and of a partial tile's way through memory (0.15 us), measured on MI355X.
+// No tile gets fewer splits than choose_splits': an fp32 sum's error grows
+// with its length.  (16384, 4096) in eight hook calls, whole calls: 426 us and
+// 3.1e-7 from 64 bits with 4 equal splits, 385 and 2.1e-7 with the tail in 18;
+// 3 splits took 367 but were 4.2e-7 off.
 // From 1024 tiles on the tail takes at most 3 splits: at (16384, 14336) 2648
 // us against 2612 with 4 (2670 with 2, 3060 without a tail), the same at 8192
 // and 4096 tokens, and with 4 the H of the full-size block check rounds so
 // that one of its 64 sampled rows parts from the oracle's at a tie (codes
 // 0.9963 alike, below its 0.999; with 2, 3, 5, 6 or 8 none does).
-// Measured before -> after (bf16, us): (16384, 4096) 335 -> 277, (32768, 3072)
-// 355 -> 294, (16384, 5120) 449 -> 436, (16384, 14336) 3060 -> 2544, (2048,
+// Measured before -> after (bf16, us): (16384, 14336) 3060 -> 2544, (2048,
 // 14336) 855 -> 535.
-HessPlan hessian_plan(int64_t n, int64_t ntiles, int splits) {
+HessPlan hessian_plan(int64_t n, int64_t ntiles, int splits, int room) {
   HessPlan best{splits, ntiles, 1};
   if (n <= 0 || ntiles <= 0 || splits < 1) return best;
   constexpr double kToken = 0.0236, kRound = 5.0, kPart = 0.15;
-  const int64_t budget = static_cast<int64_t>(splits) * ntiles;
-  const int64_t tok_max = ntiles < 512 ? 10240 : 16384;
-  const int64_t lo = ntiles >= 1024 ? splits : std::min<int64_t>(splits, std::max<int64_t>(ceil_div(3 * splits, 4), ceil_div(n, tok_max)));
-  double least = 1e300;
-  for (int64_t s1 = lo; s1 <= splits; ++s1) {
-    const int64_t rounds = ntiles * s1 / 256;
-    for (int full = 0; full < 2; ++full) {
-      // all tiles in s1 splits, or as many as fill whole rounds
-      const int64_t a = full ? 256 * rounds / s1 : ntiles;
-      const int64_t b = ntiles - a;
-      if (full && (a <= 0 || b <= 0)) continue;
-      const int64_t units1 = a * s1, kept = s1 == 1 ? 0 : units1;
-      const double t1 = static_cast<double>(ceil_div(units1, 256)) * (static_cast<double>(n) / s1 * kToken + kRound);
-      const int64_t most = !full ? 1 : ntiles >= 1024 ? std::max<int64_t>(3, s1) : 64;
-      for (int64_t s2 = full ? s1 : 1; s2 <= most; ++s2) {
-        if (full && (kept + b * s2 > budget || (s2 > s1 && n / s2 < 512))) break;
-        const int64_t units2 = full ? b * s2 : 0;
-        double t = t1 + static_cast<double>(kept + units2) * kPart;
-        if (full) t += static_cast<double>(ceil_div(units2, 256)) * (static_cast<double>(n) / s2 * kToken + kRound);
-        if (t < least) {
-          least = t;
-          best = HessPlan{static_cast<int>(s1), a, static_cast<int>(s2)};
-        }
-      }
+  const int64_t budget = static_cast<int64_t>(room) * ntiles;
+  auto round = [&](int64_t units, int64_t s) {
+    return static_cast<double>(ceil_div(units, 256)) * (static_cast<double>(n) / s * kToken + kRound);
+  };
+  // all tiles in `splits` splits, or as many as fill whole rounds and the tail in more
+  const int64_t all = ntiles * splits;
+  double least = round(all, splits) + static_cast<double>(splits == 1 ? 0 : all) * kPart;
+  const int64_t a = 256 * (all / 256) / splits, b = ntiles - a;
+  if (a <= 0 || b <= 0) return best;
+  const int64_t kept = splits == 1 ? 0 : a * splits;
+  const int64_t most = ntiles >= 1024 ? std::max<int64_t>(3, splits) : 64;
+  for (int64_t s2 = splits; s2 <= most; ++s2) {
+    if (kept + b * s2 > budget || (s2 > splits && n / s2 < 512)) break;
+    const double t = round(a * splits, splits) + round(b * s2, s2) + static_cast<double>(kept + b * s2) * kPart;
+    if (t < least) {
+      least = t;
+      best = HessPlan{splits, a, static_cast<int>(s2)};
     }
   }
   return best;
+}
+
+// Room for the partial tiles of a finer tail beside those of equal splits: one
+// split more where the tail may take it (below 1024 tiles and past one round;
+// one split's whole tiles have no partials and leave enough).
+int hessian_room(int64_t ntiles, int splits) {
+  return splits > 1 && splits < 64 && ntiles < 1024 && splits * ntiles > 256 ? splits + 1 : splits;
 }
 
 int64_t hessian_run_tokens(int64_t ntiles, int64_t cap) {
@@ -253,6 +252,12 @@ extern "C" size_t gptq_hessian_workspace_size(int64_t n, int64_t K) {
   if (n <= 0 || K <= 0 || K > (1 << 20)) return 0;
   const int64_t ntiles = plan::hessian_tiles(K);
   return static_cast<size_t>(plan::choose_splits(n, ntiles)) * plan::hessian_split_bytes(K);
+}
+
+extern "C" size_t gptq_hessian_workspace_best(int64_t n, int64_t K) {
+  if (n <= 0 || K <= 0 || K > (1 << 20)) return 0;
+  const int64_t ntiles = plan::hessian_tiles(K);
+  return static_cast<size_t>(plan::hessian_room(ntiles, plan::choose_splits(n, ntiles))) * plan::hessian_split_bytes(K);
 }
 
 extern "C" size_t gptq_hessian_workspace_min(int64_t K) {

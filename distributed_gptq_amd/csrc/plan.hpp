@@ -50,8 +50,10 @@ struct HessPlan {
   int s2;
 };
 // `splits`: what choose_splits gives; the plan's partial tiles fit in
-// splits * ntiles
-HessPlan hessian_plan(int64_t n, int64_t ntiles, int splits);
+// room * ntiles, room >= splits
+HessPlan hessian_plan(int64_t n, int64_t ntiles, int splits, int room);
+// the room of gptq_hessian_workspace_best
+int hessian_room(int64_t ntiles, int splits);
 // tokens per run when the workspace holds only `cap` splits' partial tiles
 // (fewer than choose_splits wants): runs are added to H one after the other
 int64_t hessian_run_tokens(int64_t ntiles, int64_t cap);

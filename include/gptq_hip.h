@@ -63,6 +63,11 @@ int gptq_hessian_accumulate(float* H, const void* X, int64_t n, int64_t K,
  * (its add_batch allocates nothing beyond H); for callers short of memory. */
 size_t gptq_hessian_workspace_min(int64_t K);
 
+/* gptq_hessian_workspace_size(n, K), or one split more where 16-bit inputs
+ * run faster with it: the tiles of a launch's last round are then cut into
+ * more splits.  No counterpart in the reference. */
+size_t gptq_hessian_workspace_best(int64_t n, int64_t K);
+
 /* ------------------------------------------------------- damp + factorise --
  * Hd = scale * H[perm][:, perm] (perm may be NULL); if dead_cols is non-NULL,
  * every i with Hd[i][i] == 0 gets Hd[i][i] = 1 and dead_cols[i] = 1 (else 0);

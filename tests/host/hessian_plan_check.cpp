@@ -1,6 +1,6 @@
 // Properties of plan::hessian_plan over grids of shapes: every tile gets at
-// least one split, the partial tiles fit the workspace of choose_splits, no
-// split is empty, and the splits stay within the bounds on tokens per split.
+// least one split, the partial tiles fit the room they are given, no split
+// is empty, and no tile gets fewer splits than asked for.
 #include <cinttypes>
 #include <cstdio>
 
@@ -26,21 +26,20 @@ int main() {
     for (int64_t n : ns) {
       const int64_t nt = plan::hessian_tiles(K);
       const int S = plan::choose_splits(n, nt);
-      for (int cap = S; cap >= 1; cap = cap / 2) {
-        const plan::HessPlan p = plan::hessian_plan(n, nt, cap);
-        const int64_t tail = nt - p.whole;
-        CHECK(p.s1 >= 1 && p.s1 <= cap && p.whole >= 1 && p.whole <= nt && p.s2 >= 1 && p.s2 <= 64, n, K);
-        // (one split: the first tiles have no partials)
-        const int64_t parts = (p.s1 == 1 ? 0 : p.s1 * p.whole) + p.s2 * tail;
-        CHECK(parts <= static_cast<int64_t>(cap) * nt, n, K);
-        CHECK(tail == 0 || p.s2 >= p.s1, n, K);
-        const int64_t tok = nt < 512 ? 10240 : 16384;
-        if (nt < 1024) CHECK(p.s1 == cap || plan::ceil_div(n, p.s1) <= tok, n, K);
-        else CHECK(p.s1 == cap, n, K);
-        CHECK(tail == 0 || p.s2 == p.s1 || n / p.s2 >= 512, n, K);
-      }
+      CHECK(plan::hessian_room(nt, S) >= S && plan::hessian_room(nt, S) <= 64, n, K);
+      for (int cap = S; cap >= 1; cap = cap / 2)
+        for (int room = cap; room <= plan::hessian_room(nt, cap); ++room) {
+          const plan::HessPlan p = plan::hessian_plan(n, nt, cap, room);
+          const int64_t tail = nt - p.whole;
+          CHECK(p.s1 == cap && p.whole >= 1 && p.whole <= nt && p.s2 >= 1 && p.s2 <= 64, n, K);
+          // (one split: the first tiles have no partials)
+          const int64_t parts = (p.s1 == 1 ? 0 : p.s1 * p.whole) + p.s2 * tail;
+          CHECK(parts <= static_cast<int64_t>(room) * nt, n, K);
+          CHECK(tail == 0 || p.s2 >= p.s1, n, K);
+          CHECK(tail == 0 || p.s2 == p.s1 || n / p.s2 >= 512, n, K);
+        }
     }
-  const plan::HessPlan none = plan::hessian_plan(0, 10, 3);
+  const plan::HessPlan none = plan::hessian_plan(0, 10, 3, 3);
   CHECK(none.s1 == 3 && none.whole == 10, 0, 0);
   std::printf("%d check(s) failed\n", failed);
   return failed != 0;

@@ -30,7 +30,7 @@ def test_plan_properties(tmp_path):
     (700, 776),       # partial last tiles, one split
     (1700, 5128),     # 231 tiles of one split, the last rows and columns 8 past a tile
     (3000, 6152),     # 325 tiles: 256 in one split, the tail in finer ones
-    (9000, 4104),     # two splits and a finer tail, both through partial tiles
+    (9000, 4104),     # four splits and a finer tail, both through partial tiles
     (2100, 11272),    # 1035 tiles: four whole rounds and a tail
 ])
 def test_against_fp64(n, K, dtype):
