@@ -298,6 +298,9 @@ __device__ __forceinline__ void dense_tile(const DenseArgs& a, int m0, int n0, i
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
+      // (stays in AGPRs up to here: with all blocks copied out at the start a
+      // spill of one of them was placed before the wait states)
+      asm volatile("" : "+a"(acc[i][j]));
       const f32x4& c = acc[i][j];
       const int row = 16 * i + (lane & 15);
       *(lds_u32x2*)(own + row * kRB + (((2 * j + (lane >> 5)) ^ (row & (kChunks - 1))) * 16) + ((lane >> 4) & 1) * 8) =
