@@ -36,6 +36,7 @@ import weakref
 from typing import Optional
 
 import torch
+import torch.autograd.forward_ad as fw
 import torch.nn as nn
 
 from .. import _lib as L
@@ -247,6 +248,14 @@ def _dequant_input_order(qweight, scales, zeros, g_idx, perm=None) -> torch.Tens
     return out
 
 
+def _watched() -> bool:
+    """Whether a dispatch or function mode, a tracer or a compiler looks at the
+    operators being called: kernels launched through ctypes are none."""
+    # (the compiler first: it cannot look into the others)
+    return bool(torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack()
+                or torch._C._len_torch_function_stack())
+
+
 def _linear_setup(ctx, inputs, output):
     x, qweight, scales, zeros, g_idx, bias, perm = inputs
     ctx.save_for_backward(qweight, scales, zeros, g_idx, perm)
@@ -254,15 +263,20 @@ def _linear_setup(ctx, inputs, output):
     ctx.has_bias = bias is not None
 
 
+def _plain_grad(grad) -> bool:
+    """Whether nothing beside its values is asked of a product with ``grad``:
+    it is not differentiated further (backward or forward), not a wrapper
+    without storage as under vmap, and no operator is watched."""
+    return (not _watched() and type(grad) is torch.Tensor and torch._C._has_storage(grad)
+            and not torch._C._functorch.is_functorch_wrapped_tensor(grad)
+            and not (torch.is_grad_enabled() and grad.requires_grad) and fw.unpack_dual(grad).tangent is None)
+
+
 def _grad_input(grad, qweight, scales, zeros, g_idx, perm, dtype) -> torch.Tensor:
     """grad @ W in ``dtype``, W the fp32 dequantised weights."""
-    N, K = qweight.shape[0], g_idx.numel()
-    M = grad.numel() // N if N else 0
-    # (a grad that is itself differentiated, or a wrapper without storage as
-    # under vmap, takes the torch product)
-    plain = type(grad) is torch.Tensor and torch._C._has_storage(grad) and not (
-        torch._C._functorch.is_functorch_wrapped_tensor(grad) or (torch.is_grad_enabled() and grad.requires_grad))
-    if M and plain and grad.dtype == dtype and dtype in (torch.float16, torch.bfloat16):
+    if _plain_grad(grad) and grad.numel() and grad.dtype == dtype and dtype in (torch.float16, torch.bfloat16):
+        N, K = qweight.shape[0], g_idx.numel()
+        M = grad.numel() // N
         order = perm if perm is not None and perm.numel() else None
         bits = _infer_bits(qweight, K)
         if _planes_backward(M, N, K, bits, dtype, order):
@@ -270,7 +284,9 @@ def _grad_input(grad, qweight, scales, zeros, g_idx, perm, dtype) -> torch.Tenso
             if gi is None and gs % 32 == 0 and qweight.contiguous().data_ptr() % 16 == 0:
                 gx = _ops.linear_grad_input(grad.reshape(M, N), qweight, bits, scales, zeros, K, gs, order)
                 return gx.reshape(*grad.shape[:-1], K)
-    W = _dequant_input_order(qweight, scales, zeros, g_idx, perm)
+    # (watched: the weights come from an operator, so that a trace holds their
+    # computation and not the memory that it filled)
+    W = (torch.ops.gptq.dequantize if _watched() else _dequant_input_order)(qweight, scales, zeros, g_idx, perm)
     return (grad.float() @ W).to(dtype)
 
 
@@ -287,7 +303,8 @@ def _linear_backward(ctx, grad):
 
 
 def register_ops():
-    """Define gptq::linear with its CUDA kernel and autograd (idempotent)."""
+    """Define gptq::linear with its CUDA kernel and autograd, and the fp32
+    weights of its backward as gptq::dequantize (idempotent)."""
     global _OP_LIB
     if _OP_LIB is not None:
         return
@@ -297,6 +314,8 @@ def register_ops():
     lib.define("linear(Tensor x, Tensor qweight, Tensor scales, Tensor zeros, Tensor g_idx, Tensor? bias, "
                "Tensor? perm=None) -> Tensor")
     lib.impl("linear", _linear_impl, "CUDA")
+    lib.define("dequantize(Tensor qweight, Tensor scales, Tensor zeros, Tensor g_idx, Tensor? perm=None) -> Tensor")
+    lib.impl("dequantize", _dequant_input_order, "CompositeExplicitAutograd")
     torch.library.register_autograd("gptq::linear", _linear_backward, setup_context=_linear_setup, lib=lib)
     _OP_LIB = lib
 
@@ -312,10 +331,9 @@ def _apply_linear(x, qweight, scales, zeros, g_idx, bias, perm):
     that refuses is left to gptq::linear, which raises or computes it."""
     if perm is not None and not perm.numel():
         perm = None
-    if type(x) is torch.Tensor and x.is_cuda and not torch.compiler.is_compiling() and not (
-            (torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad)))
-            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch.jit.is_tracing()):
+    if type(x) is torch.Tensor and x.is_cuda and not (
+            _watched() or (torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad)))
+            or torch._C._functorch.peek_interpreter_stack() is not None):
         K = g_idx.numel()
         if x.dtype is torch.float32 or x.numel() < DEQUANT_GEMM_ROWS * K:
             bits = _infer_bits(qweight, K)

@@ -144,6 +144,34 @@ def test_operator_routes(dtype, act):
     assert both.shape == (2, M, 4096)
 
 
+@pytest.mark.parametrize("act", [False, True])
+def test_gradient_that_is_followed(act):
+    """Forward over reverse, and a trace of a call that takes the gradient."""
+    import torch.autograd.forward_ad as fw
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from distributed_gptq_amd.models import layers
+    N, K, M = 256, 4096, 1536
+    assert layers._planes_backward(M, N, K, 4, torch.float16, None)
+    q, W = make_layer(N, K, 4, 64, act, 12)
+    x = torch.randn(M, K, device="cuda").half()
+    go, t = ((torch.randn(M, N, device="cuda") * 1e-2).half() for _ in range(2))
+
+    def grad(x, go):
+        x = x.detach().requires_grad_(True)
+        return torch.autograd.grad(q(x), x, go)[0]
+
+    with fw.dual_level():
+        gx = fw.unpack_dual(grad(x, fw.make_dual(go, t)))
+        assert gx.tangent is not None
+        check(gx.primal, go.double() @ W, go.double().abs() @ W.abs(), 6 * N)
+        check(gx.tangent, t.double() @ W, t.double().abs() @ W.abs(), 6 * N)
+    traced = make_fx(grad)(x, go)
+    del gx
+    keep = [torch.full((N, K), float("nan"), device="cuda") for _ in range(4)]  # freed memory holds no weights
+    del keep
+    check(traced(x, t), t.double() @ W, t.double().abs() @ W.abs(), 6 * N)
+
+
 def test_biases_of_the_library_product():
     """Biases that the dense kernel does not read as N values of its types
     keep the library product: its broadcast, its conversion and its errors."""
