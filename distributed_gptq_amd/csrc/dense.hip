@@ -62,7 +62,7 @@ struct DenseArgs {
   const uint16_t* B;
   uint16_t* C;
   const void* bias;     // N values or null
-  const int32_t* inexact;  // kPlaneFlags ints: all zero -> the third B plane is zero everywhere; null: one plane
+  const int32_t* inexact;  // kPlaneFlags ints: all zero -> the third B plane is zero everywhere (or null)
   int64_t lda, ldb, ldc;
   int M, N;
   int ks;               // contraction of one (A plane, B plane) segment, a multiple of kBK
@@ -88,22 +88,17 @@ __device__ __forceinline__ bool nonfinite16(uint32_t h, bool bf16) {
   return bf16 ? (h & 0x7F80u) == 0x7F80u : (h & 0x7C00u) == 0x7C00u;
 }
 
-// C[m][n] summed one term after the other from the planes' whole values: the
-// product of an infinity with a zero low plane is no term of the sum.
-template <bool kBF16>
-__device__ __noinline__ float plain_sum(const uint16_t* A, const uint16_t* B, int ks, int aplanes, int bplanes) {
-  float acc = 0.0f;
-  for (int k = 0; k < ks; ++k) {
-    float a = 0.0f, b = 0.0f;
-    for (int p = 0; p < aplanes; ++p) a += bf16_bits_to_f32(A[p * ks + k]);
-    for (int p = 0; p < bplanes; ++p) b += bf16_bits_to_f32(B[p * ks + k]);
-    acc += a * b;
-  }
-  return acc;
-}
-
 // OUT_BF16: C's type (A's own unless A is split into planes)
-template <bool kBF16, bool kOutBF16, int NBJ>
+//
+// With planes, a tile with an infinite or NaN result is multiplied again, the
+// first planes alone, and its infinite and NaN sums replace those results: an
+// infinity times a zero low plane is no term of the product, and the first
+// planes are zero, infinite or NaN where the whole values are (down to bf16's
+// subnormals).  A finite sum that only rounds to an infinity stays.  This costs
+// one plane pair more: the gradient of 1024 x 4096 x 4096, bf16, takes 172 us
+// with one infinity in each row or all NaN and 122 us without (4-bit weights;
+// summed again one element at a time it took 148 ms).
+template <bool kBF16, bool kOutBF16, bool kPlanes, int NBJ>
 __device__ __forceinline__ void dense_tile(const DenseArgs& a, int m0, int n0, int bplanes) {
   constexpr int NM = 8 * NBJ;  // MFMAs per half
   constexpr int NF = 8 + NBJ;  // fragments per half
@@ -128,43 +123,6 @@ __device__ __forceinline__ void dense_tile(const DenseArgs& a, int m0, int n0, i
   const int rowsB = a.N - n0 < 32 * NBJ ? a.N - n0 : 32 * NBJ;
   const uint32_t recA = static_cast<uint32_t>(rowsA * rowa), recB = static_cast<uint32_t>(rowsB * rowb);
 
-  // the stage being copied: byte offsets of its first column of A and B and
-  // the record counts (zero past the end: nothing is fetched).  Segment s
-  // multiplies A plane s % aplanes with B plane s / aplanes.  The descriptors
-  // stay fixed and the columns go through the scalar offset; a row past the
-  // matrix is past the records whether the hardware counts that offset in the
-  // bounds check or not.
-  const int nst = a.aplanes * bplanes * (a.ks / kBK);
-  const int seg = 2 * a.ks;
-  struct Src {
-    int oa, ob;
-    uint32_t na, nb;
-  };
-  int f_k = 0, f_a = 0, f_b = 0;  // bytes: in the segment, of the A and the B plane
-  const int f_aend = a.aplanes * seg, f_bend = bplanes * seg;
-  auto front = [&]() {
-    Src s;
-    s.oa = f_a + f_k;
-    s.ob = f_b + f_k;
-    s.na = f_b < f_bend ? recA : 0u;
-    s.nb = f_b < f_bend ? recB : 0u;
-    f_k += kRowBytes;
-    const bool wrap = f_k >= seg;
-    f_k = wrap ? 0 : f_k;
-    f_a = wrap ? f_a + seg : f_a;
-    const bool next = f_a >= f_aend;
-    f_a = next ? 0 : f_a;
-    f_b = next ? f_b + seg : f_b;
-    return s;
-  };
-  auto copy = [&](const Src& s, auto bsel, auto ksel) {
-    constexpr int B = decltype(bsel)::value, k = decltype(ksel)::value;
-    if constexpr (k < 8)
-      lds_copy16(baseA, s.na, dbuf<B>(0) + (wave + 4 * k) * 1024, voff[k], s.oa);
-    else
-      lds_copy16(baseB, s.nb, dbuf<B>(1) + (wave + 4 * (k - 8)) * 1024, voff[k], s.ob);
-  };
-
   // fragment role: lane l holds row l % 16, k 8 (l / 16) .. + 7 of a half.
   // Offsets for buffer 0, and the same 64 KB up for buffer 1 (opaque, and
   // subtracted again below), so that a read's constant part fits the
@@ -182,160 +140,220 @@ __device__ __forceinline__ void dense_tile(const DenseArgs& a, int m0, int n0, i
     }
   }
 
-  f32x4 acc[8][NBJ];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < NBJ; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  int ap = kPlanes ? a.aplanes : 1, bp = kPlanes ? bplanes : 1;
+  for (bool again = false;; again = true) {
+    // the stage being copied: byte offsets of its first column of A and B and
+    // the record counts (zero past the end: nothing is fetched).  Segment s
+    // multiplies A plane s % ap with B plane s / ap.  The descriptors
+    // stay fixed and the columns go through the scalar offset; a row past the
+    // matrix is past the records whether the hardware counts that offset in the
+    // bounds check or not.
+    const int nst = ap * bp * (a.ks / kBK);
+    const int seg = 2 * a.ks;
+    struct Src {
+      int oa, ob;
+      uint32_t na, nb;
+    };
+    int f_k = 0, f_a = 0, f_b = 0;  // bytes: in the segment, of the A and the B plane
+    const int f_aend = ap * seg, f_bend = bp * seg;
+    auto front = [&]() {
+      Src s;
+      s.oa = f_a + f_k;
+      s.ob = f_b + f_k;
+      s.na = f_b < f_bend ? recA : 0u;
+      s.nb = f_b < f_bend ? recB : 0u;
+      f_k += kRowBytes;
+      const bool wrap = f_k >= seg;
+      f_k = wrap ? 0 : f_k;
+      f_a = wrap ? f_a + seg : f_a;
+      const bool next = f_a >= f_aend;
+      f_a = next ? 0 : f_a;
+      f_b = next ? f_b + seg : f_b;
+      return s;
+    };
+    auto copy = [&](const Src& s, auto bsel, auto ksel) {
+      constexpr int B = decltype(bsel)::value, k = decltype(ksel)::value;
+      if constexpr (k < 8)
+        lds_copy16(baseA, s.na, dbuf<B>(0) + (wave + 4 * k) * 1024, voff[k], s.oa);
+      else
+        lds_copy16(baseB, s.nb, dbuf<B>(1) + (wave + 4 * (k - 8)) * 1024, voff[k], s.ob);
+    };
 
-  u32x4 fr[2][NF];  // [half][A0..A7, B0..]
-  // fragment f of half h of buffer B, in the order the MFMAs need them: A0, all of B, A1..A7
-  auto read = [&](auto bsel, auto hsel, auto fsel) {
-    constexpr int B = decltype(bsel)::value, h = decltype(hsel)::value, f = decltype(fsel)::value;
-    constexpr int idx = f == 0 ? 0 : f <= NBJ ? f + 7 : f - NBJ;
-    const lds_u8* p = idx < 8 ? (const lds_u8*)dbuf<B>(0) + (aoff[h][B] + (idx * 16 * kRowBytes - B * 65536))
-                              : (const lds_u8*)dbuf<B>(1) + (boff[h][B] + ((idx - 8) * 16 * kRowBytes - B * 65536));
-    fr[h][idx] = *(const lds_u32x4*)p;
-  };
-  // B's rows first: a lane's accumulators then run along n (C's contiguous side)
-  auto mfma = [&](auto msel) {
-    constexpr int h = decltype(msel)::value / NM, m = decltype(msel)::value % NM;
-    mfma16_asm<kBF16>(acc[m / NBJ][m % NBJ], fr[h][8 + m % NBJ], fr[h][m / NBJ]);
-  };
-  using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
+    f32x4 acc[8][NBJ];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < NBJ; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  constexpr int kFree = NF + 4;            // MFMAs before the barrier that frees the buffer
-  constexpr int kNext = 2 * NM - NF - 4;   // MFMAs before the next stage's first reads
-  constexpr int kEvery = (kNext - kFree) / NC;
-  Src src;  // of the stage being copied
-  auto stage = [&](auto bsel) {
-    constexpr int B = decltype(bsel)::value;
-    using Bn = std::integral_constant<int, 1 - B>;
-    // the scalar work for this stage's copies sits under these MFMAs (after
-    // the barrier it would hold up the MFMA pipe)
+    u32x4 fr[2][NF];  // [half][A0..A7, B0..]
+    // fragment f of half h of buffer B, in the order the MFMAs need them: A0, all of B, A1..A7
+    auto read = [&](auto bsel, auto hsel, auto fsel) {
+      constexpr int B = decltype(bsel)::value, h = decltype(hsel)::value, f = decltype(fsel)::value;
+      constexpr int idx = f == 0 ? 0 : f <= NBJ ? f + 7 : f - NBJ;
+      const lds_u8* p = idx < 8 ? (const lds_u8*)dbuf<B>(0) + (aoff[h][B] + (idx * 16 * kRowBytes - B * 65536))
+                                : (const lds_u8*)dbuf<B>(1) + (boff[h][B] + ((idx - 8) * 16 * kRowBytes - B * 65536));
+      fr[h][idx] = *(const lds_u32x4*)p;
+    };
+    // B's rows first: a lane's accumulators then run along n (C's contiguous side)
+    auto mfma = [&](auto msel) {
+      constexpr int h = decltype(msel)::value / NM, m = decltype(msel)::value % NM;
+      mfma16_asm<kBF16>(acc[m / NBJ][m % NBJ], fr[h][8 + m % NBJ], fr[h][m / NBJ]);
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+
+    constexpr int kFree = NF + 4;            // MFMAs before the barrier that frees the buffer
+    constexpr int kNext = 2 * NM - NF - 4;   // MFMAs before the next stage's first reads
+    constexpr int kEvery = (kNext - kFree) / NC;
+    Src src;  // of the stage being copied
+    auto stage = [&](auto bsel) {
+      constexpr int B = decltype(bsel)::value;
+      using Bn = std::integral_constant<int, 1 - B>;
+      // the scalar work for this stage's copies sits under these MFMAs (after
+      // the barrier it would hold up the MFMA pipe)
+      src = front();
+      sfor<0, kFree>([&](auto mc) {
+        constexpr int m = decltype(mc)::value;
+        mfma(mc);
+        if constexpr (m < NF) read(bsel, I1{}, mc);
+      });
+      sfor<0, kFree>([&](auto mc) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if constexpr (decltype(mc)::value < NF) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x004, 2, 0);
+      });
+      asm volatile("" : "+s"(src.oa), "+s"(src.ob), "+s"(src.na), "+s"(src.nb), "+s"(f_k), "+s"(f_a), "+s"(f_b));
+      __builtin_amdgcn_sched_barrier(0);
+      wait_lgkm<0>();
+      bare_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      sfor<kFree, kNext>([&](auto mc) {
+        constexpr int m = decltype(mc)::value - kFree;
+        mfma(mc);
+        if constexpr (m % kEvery == 0 && m / kEvery < NC) copy(src, bsel, std::integral_constant<int, m / kEvery>{});
+      });
+      sfor<kFree, kNext>([&](auto mc) {
+        constexpr int m = decltype(mc)::value - kFree;
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if constexpr (m % kEvery == 0 && m / kEvery < NC) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+      wait_vm<NC>();
+      bare_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      sfor<kNext, 2 * NM>([&](auto mc) {
+        constexpr int m = decltype(mc)::value - kNext;
+        mfma(mc);
+        if constexpr (m < NF) read(Bn{}, I0{}, std::integral_constant<int, m>{});
+      });
+      sfor<kNext, 2 * NM>([&](auto mc) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if constexpr (decltype(mc)::value - kNext < NF) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    };
+
     src = front();
-    sfor<0, kFree>([&](auto mc) {
-      constexpr int m = decltype(mc)::value;
-      mfma(mc);
-      if constexpr (m < NF) read(bsel, I1{}, mc);
-    });
-    sfor<0, kFree>([&](auto mc) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if constexpr (decltype(mc)::value < NF) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x004, 2, 0);
-    });
-    asm volatile("" : "+s"(src.oa), "+s"(src.ob), "+s"(src.na), "+s"(src.nb), "+s"(f_k), "+s"(f_a), "+s"(f_b));
-    __builtin_amdgcn_sched_barrier(0);
-    wait_lgkm<0>();
-    bare_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    sfor<kFree, kNext>([&](auto mc) {
-      constexpr int m = decltype(mc)::value - kFree;
-      mfma(mc);
-      if constexpr (m % kEvery == 0 && m / kEvery < NC) copy(src, bsel, std::integral_constant<int, m / kEvery>{});
-    });
-    sfor<kFree, kNext>([&](auto mc) {
-      constexpr int m = decltype(mc)::value - kFree;
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if constexpr (m % kEvery == 0 && m / kEvery < NC) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-    });
-    __builtin_amdgcn_sched_barrier(0);
+    sfor<0, NC>([&](auto kc) { copy(src, I0{}, kc); });
+    src = front();
+    sfor<0, NC>([&](auto kc) { copy(src, I1{}, kc); });
     wait_vm<NC>();
     bare_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    sfor<kNext, 2 * NM>([&](auto mc) {
-      constexpr int m = decltype(mc)::value - kNext;
-      mfma(mc);
-      if constexpr (m < NF) read(Bn{}, I0{}, std::integral_constant<int, m>{});
-    });
-    sfor<kNext, 2 * NM>([&](auto mc) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if constexpr (decltype(mc)::value - kNext < NF) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    });
-    __builtin_amdgcn_sched_barrier(0);
-  };
-
-  src = front();
-  sfor<0, NC>([&](auto kc) { copy(src, I0{}, kc); });
-  src = front();
-  sfor<0, NC>([&](auto kc) { copy(src, I1{}, kc); });
-  wait_vm<NC>();
-  bare_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  sfor<0, NF>([&](auto fc) { read(I0{}, I0{}, fc); });
-  // two stages per trip, one per buffer; a stage past the end multiplies zeros
-  // (zero-record copies), which leaves the sums unchanged
-  for (int t = 0; t < nst; t += 2) {
-    stage(I0{});
-    stage(I1{});
-  }
-  // no copy may still be writing LDS, and no wave reading it, when the
-  // epilogue reuses the buffers
-  wait_vm<0>();
-  wait_lgkm<0>();
-  bare_barrier();
-  mfma_settle();
-
-  // Epilogue through LDS, each wave in a buffer of its own: lane l, register
-  // v of block (i, j) is row 16i + l % 16, column 16j + 4 (l / 16) + v.  Rows
-  // of 32 NBJ bytes in 16-byte chunks, chunk c at c ^ (row % chunks), then
-  // 16-byte stores along C's rows.
-  constexpr int kChunks = 2 * NBJ;
-  constexpr int kRB = kChunks * 16;
-  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
-  lds_u8* own = dbuf_of(wave);
-#pragma unroll
-  for (int j = 0; j < NBJ; ++j) {
-    float b[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (a.bias) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int n = n0 + wn + 16 * j + 4 * (lane >> 4) + e;
-        b[e] = load_elem(a.bias, n < a.N ? n : a.N - 1, a.bias_dtype);
-      }
+    sfor<0, NF>([&](auto fc) { read(I0{}, I0{}, fc); });
+    // two stages per trip, one per buffer; a stage past the end multiplies zeros
+    // (zero-record copies), which leaves the sums unchanged
+    for (int t = 0; t < nst; t += 2) {
+      stage(I0{});
+      stage(I1{});
     }
+    // no copy may still be writing LDS, and no wave reading it, when the
+    // epilogue reuses the buffers
+    wait_vm<0>();
+    wait_lgkm<0>();
+    bare_barrier();
+    mfma_settle();
+    if (kPlanes && again) {  // zeros in place of what stays as it is
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      // (stays in AGPRs up to here: with all blocks copied out at the start a
-      // spill of one of them was placed before the wait states)
-      asm volatile("" : "+a"(acc[i][j]));
-      const f32x4& c = acc[i][j];
-      const int row = 16 * i + (lane & 15);
-      *(lds_u32x2*)(own + row * kRB + (((2 * j + (lane >> 5)) ^ (row & (kChunks - 1))) * 16) + ((lane >> 4) & 1) * 8) =
-          kOutBF16 ? u32x2{pack_bf16(c[0] + b[0], c[1] + b[1]), pack_bf16(c[2] + b[2], c[3] + b[3])}
-                   : u32x2{pack_f16(c[0] + b[0], c[1] + b[1]), pack_f16(c[2] + b[2], c[3] + b[3])};
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j) {
+          asm volatile("" : "+a"(acc[i][j]));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][j][e] = fabsf(acc[i][j][e]) < INFINITY ? 0.0f : acc[i][j][e];
+          asm volatile("" : "+a"(acc[i][j]));
+        }
     }
-  }
-  wave_sync();
-  constexpr int kRows = 64 / kChunks;  // rows per pass
-  const int chunk = lane % kChunks;
-  const int n = n0 + wn + 8 * chunk;
-  for (int it = 0; it < 128 / kRows; ++it) {
-    const int row = it * kRows + lane / kChunks;
-    const int m = m0 + wm + row;
-    u32x4 v = *(const lds_u32x4*)(own + row * kRB + ((chunk ^ (row & (kChunks - 1))) * 16));
-    if (m >= a.M || n >= a.N) continue;
-    if (a.inexact) {
+
+    // Epilogue through LDS, each wave in a buffer of its own: lane l, register
+    // v of block (i, j) is row 16i + l % 16, column 16j + 4 (l / 16) + v.  Rows
+    // of 32 NBJ bytes in 16-byte chunks, chunk c at c ^ (row % chunks), then
+    // 16-byte stores along C's rows.
+    // (el: the lane, opaque, so that the addresses are not kept through the loop)
+    int el = lane;
+    if constexpr (kPlanes) asm volatile("" : "+v"(el));
+    constexpr int kChunks = 2 * NBJ;
+    constexpr int kRB = kChunks * 16;
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+    lds_u8* own = dbuf_of(wave);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t h = (v[e / 2] >> (16 * (e & 1))) & 0xFFFFu;
-        if (nonfinite16(h, kOutBF16)) {
-          const float f = plain_sum<kOutBF16>(a.A + static_cast<int64_t>(m) * a.lda,
-                                              a.B + static_cast<int64_t>(n + e) * a.ldb, a.ks, a.aplanes, bplanes);
-          const uint32_t w = kOutBF16 ? f32_to_bf16_bits(f) : f32_to_f16_bits(f);
-          v[e / 2] = (e & 1) ? (v[e / 2] & 0xFFFFu) | (w << 16) : (v[e / 2] & 0xFFFF0000u) | w;
+    for (int j = 0; j < NBJ; ++j) {
+      float b[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (a.bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int n = n0 + wn + 16 * j + 4 * (el >> 4) + e;
+          b[e] = load_elem(a.bias, n < a.N ? n : a.N - 1, a.bias_dtype);
         }
       }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        // (stays in AGPRs up to here: with all blocks copied out at the start a
+        // spill of one of them was placed before the wait states)
+        asm volatile("" : "+a"(acc[i][j]));
+        f32x4 y = acc[i][j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] += b[e];
+        const int row = 16 * i + (el & 15);
+        lds_u8* at = own + row * kRB + (((2 * j + (el >> 5)) ^ (row & (kChunks - 1))) * 16) + ((el >> 4) & 1) * 8;
+        *(lds_u32x2*)at =
+            kOutBF16 ? u32x2{pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])}
+                     : u32x2{pack_f16(y[0], y[1]), pack_f16(y[2], y[3])};
+      }
     }
-    *reinterpret_cast<u32x4*>(a.C + static_cast<int64_t>(m) * a.ldc + n) = v;
+    wave_sync();
+    constexpr int kRows = 64 / kChunks;  // rows per pass
+    const int chunk = el % kChunks;
+    const int n = n0 + wn + 8 * chunk;
+    bool redo = false;
+    for (int it = 0; it < 128 / kRows; ++it) {
+      const int row = it * kRows + el / kChunks;
+      const int m = m0 + wm + row;
+      u32x4 v = *(const lds_u32x4*)(own + row * kRB + ((chunk ^ (row & (kChunks - 1))) * 16));
+      if (m >= a.M || n >= a.N) continue;
+      u32x4* out = reinterpret_cast<u32x4*>(a.C + static_cast<int64_t>(m) * a.ldc + n);
+      if constexpr (kPlanes) {
+        const u32x4 old = again ? *out : v;  // (written by this thread)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t mask = 0xFFFFu << (16 * (e & 1));
+          const bool bad = nonfinite16((old[e / 2] >> (16 * (e & 1))) & 0xFFFFu, kOutBF16);
+          redo = redo || bad;
+          if (!bad || (v[e / 2] & mask) == 0) v[e / 2] = (v[e / 2] & ~mask) | (old[e / 2] & mask);
+        }
+      }
+      *out = v;
+    }
+    // (also the barrier before the buffers are filled again)
+    if (!kPlanes || again || !__syncthreads_or(redo)) break;
+    ap = bp = 1;
   }
 }
 
 constexpr int kPlaneFlags = 256;
 
-template <bool kBF16, bool kOutBF16>
+template <bool kBF16, bool kOutBF16, bool kPlanes>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void dense_nt_k(DenseArgs a) {
   // each round of 256 workgroups (the last one with what is left) is permuted
@@ -347,7 +365,7 @@ void dense_nt_k(DenseArgs a) {
     b = r0 + x * (w >> 3) + (x < (w & 7) ? x : (w & 7)) + q;
   }
   int bplanes = a.bplanes;
-  if (a.inexact) {
+  if (kPlanes && a.inexact) {
     int any = 0;
 #pragma unroll
     for (int i = 0; i < kPlaneFlags / 64; ++i) any |= a.inexact[i * 64 + (threadIdx.x & 63)];
@@ -357,12 +375,12 @@ void dense_nt_k(DenseArgs a) {
   int tm, tn;
   if (b < a.full) {
     dense_coords(b, a.ntm, a.ntn, tm, tn);
-    dense_tile<kBF16, kOutBF16, 8>(a, tm * 256, tn * 256, bplanes);
+    dense_tile<kBF16, kOutBF16, kPlanes, 8>(a, tm * 256, tn * 256, bplanes);
   } else {
     const int h = b - a.full;
     dense_coords(a.full + h / 2, a.ntm, a.ntn, tm, tn);
     const int n0 = tn * 256 + (h & 1) * 128;
-    if (n0 < a.N) dense_tile<kBF16, kOutBF16, 4>(a, tm * 256, n0, bplanes);
+    if (n0 < a.N) dense_tile<kBF16, kOutBF16, kPlanes, 4>(a, tm * 256, n0, bplanes);
   }
 }
 
@@ -432,12 +450,14 @@ extern "C" int gptq_matmul_nt(const void* A, int64_t lda, const void* B, int64_t
   a.full = static_cast<int>(rest <= 128 ? tiles - rest : tiles);
   const dim3 grid(static_cast<unsigned>(a.full + 2 * (tiles - a.full)));
   hipStream_t st = as_hip(stream);
-  if (dtype == GPTQ_BF16 && out_dtype == GPTQ_BF16)
-    hipLaunchKernelGGL((dense_nt_k<true, true>), grid, dim3(256), 0, st, a);
+  if (bplanes > 1 && out_dtype == GPTQ_BF16)
+    hipLaunchKernelGGL((dense_nt_k<true, true, true>), grid, dim3(256), 0, st, a);
+  else if (bplanes > 1)
+    hipLaunchKernelGGL((dense_nt_k<true, false, true>), grid, dim3(256), 0, st, a);
   else if (dtype == GPTQ_BF16)
-    hipLaunchKernelGGL((dense_nt_k<true, false>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((dense_nt_k<true, true, false>), grid, dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL((dense_nt_k<false, false>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((dense_nt_k<false, false, false>), grid, dim3(256), 0, st, a);
   return check_launch("matmul_nt");
 }
 

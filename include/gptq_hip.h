@@ -298,8 +298,9 @@ int gptq_linear_perm_noalloc(const void* x, int x_dtype, int64_t M,
  * With planes, A and B are bf16 and hold `aplanes` (1 or 2) and 3 matrices of
  * K columns side by side; every plane of A meets every plane of B.  `inexact`
  * (256 ints, from gptq_dequant_planes_t) tells the kernel whether B's third
- * plane is used; results that come out infinite or NaN are summed again term
- * by term, as the unsplit product would. */
+ * plane is used (NULL: it is).  Tiles with infinite or NaN results are
+ * multiplied again without the low planes, so that an infinity meets no zero
+ * that the unsplit product does not have. */
 int gptq_matmul_nt(const void* A, int64_t lda, const void* B, int64_t ldb,
                    int dtype, int64_t M, int64_t N, int64_t K, int aplanes,
                    int bplanes, const int32_t* inexact, const void* bias,

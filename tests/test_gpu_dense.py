@@ -116,6 +116,64 @@ def test_input_gradient_of_infinities(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("M,N,K", [(300, 192, 544), (2304, 192, 3840)])  # tiles as halves; 135 whole tiles
+def test_tiles_with_infinities(M, N, K, dtype):
+    """Infinite and NaN gradients and scales, and sums that are too large for
+    the type, in some tiles: the unsplit product's infinities and NaNs there,
+    every other value as without them."""
+    from distributed_gptq_amd import _ops
+    q, _ = make_layer(N, K, 4, 32, True, 6)
+    go = (torch.randn(M, N, device="cuda") * 1e-2).to(dtype)
+    clean = _ops.linear_grad_input(go, q.qweight, 4, q.scales, q.zeros, K, 32, q.perm)
+    go[5, 7], go[6], go[M - 1, N - 1], go[M // 2, 3] = float("inf"), -float("inf"), float("inf"), float("nan")
+    go[M // 2, :2] = 0
+    q.scales[N // 2, 2], q.scales[1, 3] = float("inf"), float("-inf")
+    go[9] = torch.finfo(dtype).max if dtype == torch.float16 else 1e30  # (bf16 has fp32's range)
+    W = q.unpack_weights()
+    ref32 = go.float() @ W
+    # (row 9's sums next to the largest value round to it or past it)
+    edge = (ref32[9].abs() / torch.finfo(dtype).max - 1).abs() < 0.01
+    gx = _ops.linear_grad_input(go, q.qweight, 4, q.scales, q.zeros, K, 32, q.perm)
+    ref = ref32.to(dtype)
+    gx[9, edge], ref[9, edge] = 0, 0
+    assert torch.equal(torch.isnan(gx), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert inf[5].any() and inf[:, 64:].any() and torch.equal(torch.isinf(gx), inf) and torch.equal(gx[inf], ref[inf])
+    if dtype == torch.float16:
+        assert (inf[9] & torch.isfinite(ref32[9])).any()
+    same = torch.isfinite(ref)
+    same[9] = False
+    # (a group's third plane is used now: its zeros change no sum)
+    assert same.any() and torch.equal(gx[same], clean[same])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_infinite_gradients_cost_no_more_than_a_second_product(dtype):
+    from distributed_gptq_amd import _ops
+    M, N, K = 1024, 2048, 4096
+    q, _ = make_layer(N, K, 4, 128, False, 7)
+
+    def us(go):
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            _ops.linear_grad_input(go, q.qweight, 4, q.scales, q.zeros, K, 128)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 1e3)
+        return min(times)
+
+    go = (torch.randn(M, N, device="cuda") * 1e-2).to(dtype)
+    finite = us(go)
+    go[:, 5] = float("inf")
+    one = us(go)
+    go[:] = float("nan")
+    every = us(go)
+    assert max(one, every) <= 2 * finite, (finite, one, every)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("act", [False, True])
 def test_operator_routes(dtype, act):
     """Forward on the dense kernel, backward on the planes, through the
