@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import re
 import threading
 
 import torch  # noqa: F401  (must precede the library load, see module doc)
@@ -131,6 +132,15 @@ def check(status: int, fn: str):
     if status == ERR_DTYPE:
         raise TypeError(f"{fn}: {msg}")
     raise GPTQLibraryError(status, fn, msg)
+
+
+def reraise(e: RuntimeError):
+    """Raise ``e``, an error of a native torch operator, as ``check`` raises
+    the status that its message tells of (if it does)."""
+    m = re.match(r"(\w+) failed \(status (\d+)\): (.*)", str(e), re.S)
+    if m is None:
+        raise e
+    raise GPTQLibraryError(int(m[2]), m[1], m[3]) from e
 
 
 def call(name: str, *args):

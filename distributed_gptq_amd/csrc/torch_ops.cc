@@ -26,10 +26,12 @@ int dtype_code(at::ScalarType t) {
 at::Tensor linear_rows(const at::Tensor& x, const at::Tensor& qweight, const at::Tensor& scales,
                        const at::Tensor& zeros, const std::optional<at::Tensor>& bias,
                        const std::optional<at::Tensor>& perm, int64_t bits, int64_t group_size, int64_t K) {
-  TORCH_CHECK(x.is_cuda() && qweight.device() == x.device() && scales.device() == x.device() &&
-                  zeros.device() == x.device() && (!bias || bias->device() == x.device()) &&
-                  (!perm || perm->device() == x.device()),
-              "gptq::linear_rows: expected GPU tensors on one device");
+  // what is refused is a ValueError or a TypeError, which the caller leaves to
+  // gptq::linear; everything else is a failure
+  TORCH_CHECK_VALUE(x.is_cuda() && qweight.device() == x.device() && scales.device() == x.device() &&
+                        zeros.device() == x.device() && (!bias || bias->device() == x.device()) &&
+                        (!perm || perm->device() == x.device()),
+                    "gptq::linear_rows: expected GPU tensors on one device");
   TORCH_CHECK_VALUE(K > 0 && x.dim() > 0 && x.size(-1) == K && qweight.dim() == 2 && scales.dim() == 2 &&
                         zeros.sizes() == scales.sizes() && scales.size(0) == qweight.size(0) &&
                         qweight.scalar_type() == at::kByte && qweight.is_contiguous() &&

@@ -32,6 +32,7 @@ does, and reorders the codes again.
 from __future__ import annotations
 
 import math
+import warnings
 import weakref
 from typing import Optional
 
@@ -323,12 +324,33 @@ def register_ops():
 register_ops()
 
 
+_rows_op = None  # gptq::linear_rows; False where its library cannot be loaded
+
+
+def _native_rows():
+    """gptq::linear_rows, loaded at the first call that can use it, or False:
+    an install without its library (not built, or built against another torch)
+    is served by gptq::linear, which needs libgptq_hip.so alone."""
+    global _rows_op
+    if _rows_op is None:
+        try:
+            L.load_torch_ops()
+            _rows_op = torch.ops.gptq.linear_rows.default
+        except (ImportError, OSError, AttributeError) as e:
+            L.load()  # (without libgptq_hip.so no call can be served)
+            warnings.warn(f"the native operator is not available ({e}); calls on few rows take about 16 us more of "
+                          "host time through gptq::linear", RuntimeWarning, stacklevel=2)
+            _rows_op = False
+    return _rows_op
+
+
 def _apply_linear(x, qweight, scales, zeros, g_idx, bias, perm):
     """gptq::linear, called by the modules.  The common serving call (no
     gradient, few rows or fp32 x, contiguous groups, no dispatch mode or
     tracing that would look for the operator) goes to the native
-    gptq::linear_rows: 8 us of host time a call instead of 25 us.  Whatever
-    that refuses is left to gptq::linear, which raises or computes it."""
+    gptq::linear_rows: 8 us of host time a call instead of 25 us.  What it
+    refuses (ValueError, TypeError) is left to gptq::linear, which raises or
+    computes it; a failure is not run again."""
     if perm is not None and not perm.numel():
         perm = None
     if type(x) is torch.Tensor and x.is_cuda and not (
@@ -338,21 +360,17 @@ def _apply_linear(x, qweight, scales, zeros, g_idx, bias, perm):
         if x.dtype is torch.float32 or x.numel() < DEQUANT_GEMM_ROWS * K:
             bits = _infer_bits(qweight, K)
             gs, gi = _group_layout(g_idx, K, scales.shape[1], perm)
-            if gi is None:
-                global _rows_op
-                if _rows_op is None:
-                    L.load_torch_ops()
-                    _rows_op = torch.ops.gptq.linear_rows.default
+            rows = gi is None and (_rows_op or _native_rows())
+            if rows:
                 try:
-                    return _rows_op(x, qweight, scales, zeros, bias, perm, bits, gs, K)
-                except (ValueError, TypeError, RuntimeError):
+                    return rows(x, qweight, scales, zeros, bias, perm, bits, gs, K)
+                except (ValueError, TypeError):
                     pass
+                except RuntimeError as e:
+                    L.reraise(e)
     if perm is not None:
         return torch.ops.gptq.linear(x, qweight, scales, zeros, g_idx, bias, perm)
     return torch.ops.gptq.linear(x, qweight, scales, zeros, g_idx, bias)
-
-
-_rows_op = None
 
 
 # -------------------------------------------------------- QuantizedLinear --

@@ -82,3 +82,61 @@ def test_calls_left_to_the_operator():
         q.qweight.data = q.qweight[:, :-1].contiguous()
         with pytest.raises(ValueError):
             q(x)
+
+
+@pytest.mark.parametrize("error", [ImportError("not built"), OSError("undefined symbol"), None])
+def test_without_the_native_library(monkeypatch, error, tmp_path):
+    """An install with libgptq_hip.so alone serves through gptq::linear."""
+    from distributed_gptq_amd import _lib
+    from distributed_gptq_amd.models import layers
+
+    def load(path=None):
+        raise error
+    monkeypatch.setattr(layers, "_rows_op", None)
+    if error is not None:
+        monkeypatch.setattr(_lib, "load_torch_ops", load)
+    else:  # the loader's own answer to a missing file
+        monkeypatch.setattr(_lib, "_torch_ops", False)
+        loader, missing = _lib.load_torch_ops, str(tmp_path / "libgptq_torch.so")
+        monkeypatch.setattr(_lib, "load_torch_ops", lambda: loader(missing))
+    q = layer(256, 512, 4, 128)
+    x = torch.randn(8, 512, device="cuda").half()
+    with torch.no_grad():
+        with pytest.warns(RuntimeWarning, match="native operator is not available"):
+            y = q(x)
+        assert torch.equal(y, general(q, x)) and torch.equal(q(x), y)
+    assert layers._rows_op is False
+
+
+def test_failures_are_raised_and_refusals_left(monkeypatch):
+    """A failure of the native operator is not run again through gptq::linear;
+    a status is the library's own error type."""
+    from distributed_gptq_amd import _lib
+    from distributed_gptq_amd.models import layers
+    q = layer(256, 512, 4, 128)
+    x = torch.randn(8, 512, device="cuda").half()
+    with torch.no_grad():
+        y = q(x)
+        for error in (ValueError("refused"), TypeError("refused")):
+            def refuse(*a, error=error):
+                raise error
+            monkeypatch.setattr(layers, "_rows_op", refuse)
+            assert torch.equal(q(x), y)
+        monkeypatch.setattr(torch.ops.gptq, "linear", None)  # not called from here on
+        for error, kind, text in (
+                (torch.OutOfMemoryError("no memory"), torch.OutOfMemoryError, "no memory"),
+                (RuntimeError("a device error"), RuntimeError, "a device error"),
+                (RuntimeError("gptq_linear_ws failed (status 5): launch"), _lib.GPTQLibraryError, "launch")):
+            def fail(*a, error=error):
+                raise error
+            monkeypatch.setattr(layers, "_rows_op", fail)
+            with pytest.raises(kind, match=text) as got:
+                q(x)
+            assert kind is not _lib.GPTQLibraryError or got.value.status == _lib.ERR_LAUNCH
+
+
+def test_tensors_on_two_devices_are_refused():
+    q = layer(256, 512, 4, 128)
+    q.scales.data = q.scales.cpu()
+    with torch.no_grad(), pytest.raises(RuntimeError, match="GPU tensor"):
+        q(torch.randn(8, 512, device="cuda").half())
