@@ -354,7 +354,9 @@ def _apply_linear(x, qweight, scales, zeros, g_idx, bias, perm):
     if perm is not None and not perm.numel():
         perm = None
     if type(x) is torch.Tensor and x.is_cuda and not (
-            _watched() or (torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad)))
+            _watched() or (torch.is_grad_enabled() and (
+                x.requires_grad or scales.requires_grad or zeros.requires_grad
+                or (bias is not None and bias.requires_grad)))
             or torch._C._functorch.peek_interpreter_stack() is not None):
         K = g_idx.numel()
         if x.dtype is torch.float32 or x.numel() < DEQUANT_GEMM_ROWS * K:

@@ -140,3 +140,16 @@ def test_tensors_on_two_devices_are_refused():
     q.scales.data = q.scales.cpu()
     with torch.no_grad(), pytest.raises(RuntimeError, match="GPU tensor"):
         q(torch.randn(8, 512, device="cuda").half())
+
+
+def test_scales_that_require_a_gradient():
+    """No gradient reaches them, but the call is part of the graph."""
+    q = layer(256, 512, 4, 128, bias=False)
+    x = torch.randn(8, 512, device="cuda").half()
+    assert not q(x).requires_grad
+    for t in (q.scales, q.zeros):
+        t.requires_grad_(True)
+        assert q(x).requires_grad
+        with torch.no_grad():
+            assert not q(x).requires_grad
+        t.requires_grad_(False)
