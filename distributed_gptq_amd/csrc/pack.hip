@@ -305,7 +305,8 @@ __global__ __launch_bounds__(256) void dequant_planes_t_k(const uint8_t* __restr
   for (int i = tid; i < planes * 128 * 8; i += 256) {
     const int ch = i & 7, k = (i >> 3) & 127, p = i >> 10;
     if (k0 + k >= K) continue;
-    const int64_t row = perm ? perm[k0 + k] : k0 + k;
+    // out-of-range columns are clamped so that no store leaves the array
+    const int64_t row = perm ? std::min<int64_t>(std::max<int64_t>(perm[k0 + k], 0), K - 1) : k0 + k;
     *reinterpret_cast<uint4*>(out + row * 3 * N + p * N + n0 + ch * 8) = *reinterpret_cast<const uint4*>(&t[p][k][ch * 8]);
   }
 }

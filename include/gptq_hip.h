@@ -309,11 +309,12 @@ int gptq_matmul_nt(const void* A, int64_t lda, const void* B, int64_t ldb,
 
 /* The weights of gptq_dequant (contiguous groups of group_size columns; bits
  * 0: one code per byte) transposed and split exactly into three bf16 planes:
- * out row k (row perm[k] with perm) holds column k's N weights three times,
- * 3 N values.  N % 64 == 0, K % 32 == 0, group_size % 32 == 0, packed and out
- * 16-byte aligned.  flags (256 ints) are written: all zero when two planes
- * hold every weight, the third then is not written.  For the input gradient
- * of F.linear(x, unpack_weights()) (models/layers.py:155-157). */
+ * out row k (row perm[k] with perm, clamped to [0, K)) holds column k's N
+ * weights three times, 3 N values.  N % 64 == 0, K % 32 == 0,
+ * group_size % 32 == 0, packed and out 16-byte aligned.  flags (256 ints) are
+ * written: all zero when two planes hold every weight, the third then is not
+ * written.  For the input gradient of F.linear(x, unpack_weights())
+ * (models/layers.py:155-157). */
 int gptq_dequant_planes_t(const uint8_t* packed, int bits, const void* scales,
                           const void* zeros, int sz_dtype, int group_size,
                           int64_t ngroups, int64_t N, int64_t K,
