@@ -1,5 +1,7 @@
 """The native gptq::linear_rows behind the modules: the same bits as
 gptq::linear over the forms a call can take, and the calls it leaves to it."""
+import warnings
+
 import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
@@ -143,13 +145,19 @@ def test_tensors_on_two_devices_are_refused():
 
 
 def test_scales_that_require_a_gradient():
-    """No gradient reaches them, but the call is part of the graph."""
+    """No gradient reaches them, but the call is part of the graph, and its
+    backward is gptq::linear's (the native operator has none: it would warn)."""
     q = layer(256, 512, 4, 128, bias=False)
     x = torch.randn(8, 512, device="cuda").half()
     assert not q(x).requires_grad
     for t in (q.scales, q.zeros):
         t.requires_grad_(True)
-        assert q(x).requires_grad
+        y = q(x)
+        assert y.requires_grad
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            y.float().sum().backward()
+        assert t.grad is None
         with torch.no_grad():
             assert not q(x).requires_grad
         t.requires_grad_(False)
