@@ -55,16 +55,18 @@ int choose_splits(int64_t n, int64_t ntiles) {
 // round.  By the time of a round (23.6 ns a token, 5 us of start and drain)
 // and of a partial tile's way through memory (0.15 us), measured on MI355X.
 // No tile gets fewer splits than choose_splits': an fp32 sum's error grows
-// with its length.  (16384, 4096) in eight hook calls, whole calls: 426 us and
-// 3.1e-7 from 64 bits with 4 equal splits, 385 and 2.1e-7 with the tail in 18;
-// 3 splits took 367 but were 4.2e-7 off.
-// From 1024 tiles on the tail takes at most 3 splits: at (16384, 14336) 2648
-// us against 2612 with 4 (2670 with 2, 3060 without a tail), the same at 8192
-// and 4096 tokens, and with 4 the H of the full-size block check rounds so
-// that one of its 64 sampled rows parts from the oracle's at a tie (codes
-// 0.9963 alike, below its 0.999; with 2, 3, 5, 6 or 8 none does).
-// Measured before -> after (bf16, us): (16384, 14336) 3060 -> 2544, (2048,
-// 14336) 855 -> 535.
+// with its length (K = 4096, 16384 tokens, H's error against 64 bits, the same
+// for three seeds: 2.3e-7 with 4 equal splits, 1.8e-7 with the tail in 18;
+// K = 14336, 8192 tokens: 5.2e-7 in one, 4.2e-7 with the tail in 3).
+// From 1024 tiles on, the fewest tail splits within 1% of the least time are
+// taken: the model is no better than that there.  Measured over 40 pairs of K
+// = 11520 ... 20480 and n = 1024 ... 16384, each with up to 14 tails: the
+// least modelled time is 0.13% (at most 1.2%) behind the fastest tail, the
+// fewest splits within 1% are 0.16% (1.1%) behind it with a third fewer
+// partial tiles.  Below (43 pairs), these would be 0.46% (2.3%) behind, and
+// the least modelled time is 0.29% (1.7%).
+// Equal splits -> this plan, whole calls (bf16, us): (16384, 14336) 3110 ->
+// 2600, (2048, 14336) 843 -> 530, (16384, 4096) 334 -> 299.
 HessPlan hessian_plan(int64_t n, int64_t ntiles, int splits, int room) {
   HessPlan best{splits, ntiles, 1};
   if (n <= 0 || ntiles <= 0 || splits < 1) return best;
@@ -75,20 +77,26 @@ HessPlan hessian_plan(int64_t n, int64_t ntiles, int splits, int room) {
   };
   // all tiles in `splits` splits, or as many as fill whole rounds and the tail in more
   const int64_t all = ntiles * splits;
-  double least = round(all, splits) + static_cast<double>(splits == 1 ? 0 : all) * kPart;
   const int64_t a = 256 * (all / 256) / splits, b = ntiles - a;
   if (a <= 0 || b <= 0) return best;
   const int64_t kept = splits == 1 ? 0 : a * splits;
-  const int64_t most = ntiles >= 1024 ? std::max<int64_t>(3, splits) : 64;
-  for (int64_t s2 = splits; s2 <= most; ++s2) {
-    if (kept + b * s2 > budget || (s2 > splits && n / s2 < 512)) break;
-    const double t = round(a * splits, splits) + round(b * s2, s2) + static_cast<double>(kept + b * s2) * kPart;
-    if (t < least) {
-      least = t;
-      best = HessPlan{splits, a, static_cast<int>(s2)};
-    }
-  }
-  return best;
+  const double equal = round(all, splits) + static_cast<double>(splits == 1 ? 0 : all) * kPart;
+  auto allowed = [&](int64_t s2) {
+    return s2 <= 64 && kept + b * s2 <= budget && (s2 == splits || n / s2 >= 512);
+  };
+  auto time = [&](int64_t s2) {
+    return round(a * splits, splits) + round(b * s2, s2) + static_cast<double>(kept + b * s2) * kPart;
+  };
+  double least = equal;
+  for (int64_t s2 = splits; allowed(s2); ++s2) least = std::min(least, time(s2));
+  const double within = ntiles >= 1024 ? 1.01 * least : least;
+  if (equal <= within) return best;
+  int64_t s2 = splits;
+  while (time(s2) > within) ++s2;
+  // (whole 32s of tokens a split: the last of many could be left without any)
+  auto used = [&](int64_t s) { return ceil_div(n, ceil_div(ceil_div(n, s), 32) * 32); };
+  while (s2 > splits && used(s2) < s2) --s2;
+  return HessPlan{splits, a, static_cast<int>(s2)};
 }
 
 // Room for the partial tiles of a finer tail beside those of equal splits: one

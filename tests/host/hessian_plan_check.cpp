@@ -1,6 +1,6 @@
 // Properties of plan::hessian_plan over grids of shapes: every tile gets at
-// least one split, the partial tiles fit the room they are given, no split
-// is empty, and no tile gets fewer splits than asked for.
+// least one split, the partial tiles fit the room they are given, no split of
+// a finer tail is empty, and no tile gets fewer splits than asked for.
 #include <cinttypes>
 #include <cstdio>
 
@@ -18,9 +18,9 @@ static int failed = 0;
   } while (0)
 
 int main() {
-  const int64_t Ks[] = {8, 64, 256, 264, 768, 1024, 2048, 3072, 4096, 4104, 5120, 6152, 8192, 11008, 11272, 13824,
+  const int64_t Ks[] = {8, 64, 256, 264, 752, 768, 1024, 2048, 3072, 4096, 4104, 5120, 6152, 8192, 11008, 11272, 13824,
                         14336, 28672, 65536, 1 << 20};
-  const int64_t ns[] = {1, 31, 32, 100, 511, 512, 1023, 1024, 2048, 4097, 8229, 10277, 16384, 27685, 28709, 32768,
+  const int64_t ns[] = {1, 31, 32, 100, 511, 512, 1023, 1024, 2048, 4097, 8229, 10277, 16384, 27685, 28709, 32768, 44038,
                         65536, 262144, 1 << 24, INT64_MAX};
   for (int64_t K : Ks)
     for (int64_t n : ns) {
@@ -37,6 +37,8 @@ int main() {
           CHECK(parts <= static_cast<int64_t>(room) * nt, n, K);
           CHECK(tail == 0 || p.s2 >= p.s1, n, K);
           CHECK(tail == 0 || p.s2 == p.s1 || n / p.s2 >= 512, n, K);
+          const int64_t per = ((n / p.s2 + (n % p.s2 != 0)) + 31) / 32 * 32;  // a tail split's tokens
+          CHECK(tail == 0 || p.s2 == p.s1 || (p.s2 - 1) * per < n, n, K);
         }
     }
   const plan::HessPlan none = plan::hessian_plan(0, 10, 3, 3);
