@@ -105,10 +105,12 @@ def _group_layout(g_idx: torch.Tensor, K: int, ngroups: int, perm: Optional[torc
 
 # Rows of x from which the weights are dequantised once (to x's dtype) and
 # multiplied as a dense product instead of the fused kernels, which decode
-# every weight once per 128 rows.  Measured on MI355X (4-bit, fp16/bf16, the
-# Llama-3-8B and 13B layer shapes, the product in the library): at 384 rows
-# the two are even or the product wins, at 512 it wins everywhere, at 16384
-# rows by 3.4-3.7x.
+# every weight once per 128 rows.  Measured on MI355X (4-bit, us, fused /
+# dequantised, bf16; fp16 is within 10%): 28672 x 4096 at 320, 384 and 448 rows
+# 148 / 146, 152 / 155, 356 / 154; 13824 x 5120 119 / 86, 120 / 90, 222 / 97;
+# 4096 x 14336 89 / 92, 89 / 92, 147 / 102; 5120 x 5120 44 / 49, 44 / 49,
+# 104 / 53; 5120 x 13824 94 / 102, 93 / 104, 261 / 118; 4096 x 4096 35 / 49,
+# 35 / 49, 47 / 49 (at 1024 rows 93 / 53).
 DEQUANT_GEMM_ROWS = 384
 
 
@@ -170,11 +172,14 @@ def _dense_rounds(M: int, N: int) -> float:
 
 def _dense_forward(M: int, N: int, K: int) -> bool:
     """Whether x @ W^T on many rows runs on the dense kernel: where its tiles
-    fill at least 65% of the rounds they take.  Measured (bf16, us, against
-    the library GEMM with fp32 output and the cast; M, N, K): 2048 x 28672 x
-    4096 (0.88 filled) 415 / 565, 512 x 28672 x 4096 (0.88) 88 / 118, 2048 x
-    4096 x 4096 (0.91) 58 / 72; below, 2048 x 5120 x 5120 (0.63) 108 / 101,
-    1024 x 4096 x 14336 (0.45) 157 / 120."""
+    fill at least 65% of the rounds they take.  Measured (us, bf16 and fp16,
+    against the library GEMM with fp32 output and the cast; M, N, K): 2048 x
+    28672 x 4096 (0.99 filled) 350 / 464 and 366 / 475, 512 x 28672 x 4096
+    (0.88) 87 / 120 and 91 / 129, 1024 x 13824 x 5120 (0.84) 101 / 123 and 107
+    / 129, 2048 x 6144 x 4096 (0.75) 79 / 91 and 84 / 96, 384 x 28672 x 4096
+    (0.66) 85 / 98 and 88 / 100.  At 0.54 to 0.62 it is 4% ahead or more (2048
+    x 5120 x 5120 (0.62) 92 / 96 and 96 / 101), at 0.45 and less behind: 1024 x
+    4096 x 14336 139 / 123 and 139 / 124, 512 x 4096 x 4096 (0.23) 44 / 30."""
     if K % 64 or N % 8 or max(M, N) > 1 << 24 or K >= 1 << 22:  # the kernel's ranges
         return False
     return M * N >= 0.65 * _dense_rounds(M, N) * 256 * 65536
