@@ -347,6 +347,7 @@ __device__ __forceinline__ void dense_tile(const DenseArgs& a, int m0, int n0, i
     }
     // (also the barrier before the buffers are filled again)
     if (!kPlanes || again || !__syncthreads_or(redo)) break;
+    wait_vm<0>();  // the stores, which the waits for copies would count
     ap = bp = 1;
   }
 }
