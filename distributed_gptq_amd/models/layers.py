@@ -99,7 +99,7 @@ def _group_layout(g_idx: torch.Tensor, K: int, ngroups: int, perm: Optional[torc
             res = (gs, None)
         else:
             res = (math.ceil(K / ngroups), gi.contiguous())
-    _layout_cache[key] = (weakref.ref(g_idx, lambda _r, k=key: _layout_cache.pop(k, None)), stamp, res)
+    _layout_cache[key] = (weakref.ref(g_idx, lambda _r, k=key, c=_layout_cache: c.pop(k, None)), stamp, res)
     return res
 
 
