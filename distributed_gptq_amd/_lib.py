@@ -152,6 +152,8 @@ def call(name: str, *args):
 
 def require_gpu(t: torch.Tensor | None = None):
     """The product path runs on the GPU only; fail loudly otherwise."""
+    if t is not None and t.is_cuda and _handle is not None:
+        return  # (a GPU tensor: there is a GPU; the queries below take 1 us each)
     if not torch.cuda.is_available():
         raise RuntimeError("distributed_gptq_amd needs an AMD GPU (gfx950) and has no CPU fallback")
     if t is not None and t.device.type != "cuda":

@@ -180,6 +180,8 @@ def _dense_forward(M: int, N: int, K: int) -> bool:
     (0.66) 85 / 98 and 88 / 100.  At 0.54 to 0.62 it is 4% ahead or more (2048
     x 5120 x 5120 (0.62) 92 / 96 and 96 / 101), at 0.45 and less behind: 1024 x
     4096 x 14336 139 / 123 and 139 / 124, 512 x 4096 x 4096 (0.23) 44 / 30."""
+    if M * N < 0.65 * 0.55 * 256 * 65536:  # not 65% of the shortest round
+        return False
     if K % 64 or N % 8 or max(M, N) > 1 << 24 or K >= 1 << 22:  # the kernel's ranges
         return False
     return M * N >= 0.65 * _dense_rounds(M, N) * 256 * 65536
@@ -215,9 +217,10 @@ def _linear_impl(x, qweight, scales, zeros, g_idx, bias, perm=None):
     if rows >= DEQUANT_GEMM_ROWS and x.dtype in (torch.float16, torch.bfloat16):
         # the reference's fallback F.linear(x, unpack_weights(), bias)
         # (models/layers.py:155-157), with the weights rounded to x's dtype once
+        N = qweight.shape[0]
         W = _ops.dequant(qweight, bits, scales, zeros, K, g_idx=gi, group_size=gs, dtype=x.dtype)
         if perm is not None:
-            if rows < W.shape[0]:
+            if rows < N:
                 x = x.index_select(-1, perm.long())
             else:
                 Wi = torch.empty_like(W)
@@ -227,16 +230,17 @@ def _linear_impl(x, qweight, scales, zeros, g_idx, bias, perm=None):
         # x's dtype (a 16-bit product may otherwise reduce split-K partials in
         # 16 bits, torch's allow_*_reduced_precision_reduction default)
         x2 = x.reshape(-1, K)
-        # (other biases keep the library's broadcast, conversion and errors)
-        plain_bias = bias is None or (bias.shape == W.shape[:1] and bias.device == x.device and
-                                      bias.dtype in (torch.float32, torch.float16, torch.bfloat16))
-        if plain_bias and _dense_forward(rows, W.shape[0], K):
-            return _ops.matmul_nt(x2, W, bias).reshape(*x.shape[:-1], W.shape[0])
+        # (biases that are not N values of these types keep the library's
+        # broadcast, conversion and errors)
+        if _dense_forward(rows, N, K) and (bias is None or (
+                bias.shape == (N,) and bias.device == x.device and
+                bias.dtype in (torch.float32, torch.float16, torch.bfloat16))):
+            return _ops.matmul_nt(x2, W, bias).reshape(*x.shape[:-1], N)
         if bias is None:
             y = torch.mm(x2, W.t(), out_dtype=torch.float32)
         else:
             y = torch.addmm(bias.to(torch.float32), x2, W.t(), out_dtype=torch.float32)
-        return y.to(x.dtype).reshape(*x.shape[:-1], W.shape[0])
+        return y.to(x.dtype).reshape(*x.shape[:-1], N)
     return _ops.linear(x, qweight, bits, scales, zeros, K, g_idx=gi, group_size=gs, bias=bias, perm=perm)
 
 
@@ -258,7 +262,7 @@ def _watched() -> bool:
     """Whether a dispatch or function mode, a tracer or a compiler looks at the
     operators being called: kernels launched through ctypes are none."""
     # (the compiler first: it cannot look into the others)
-    return bool(torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack()
+    return bool(torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack()
                 or torch._C._len_torch_function_stack())
 
 
@@ -358,13 +362,17 @@ def _apply_linear(x, qweight, scales, zeros, g_idx, bias, perm):
     computes it; a failure is not run again."""
     if perm is not None and not perm.numel():
         perm = None
-    if type(x) is torch.Tensor and x.is_cuda and not (
-            _watched() or (torch.is_grad_enabled() and (
-                x.requires_grad or scales.requires_grad or zeros.requires_grad
-                or (bias is not None and bias.requires_grad)))
-            or torch._C._functorch.peek_interpreter_stack() is not None):
-        K = g_idx.numel()
-        if x.dtype is torch.float32 or x.numel() < DEQUANT_GEMM_ROWS * K:
+    # (the number of rows first: calls of many rows, which take gptq::linear, pay
+    # for little more than that)
+    if (type(x) is torch.Tensor and not (torch.compiler.is_compiling() or torch._C._is_tracing())
+            and (x.dtype is torch.float32 or x.numel() < DEQUANT_GEMM_ROWS * g_idx.numel())):
+        if x.is_cuda and not (
+                (torch.is_grad_enabled() and (
+                    x.requires_grad or scales.requires_grad or zeros.requires_grad
+                    or (bias is not None and bias.requires_grad)))
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch._C._functorch.peek_interpreter_stack() is not None):
+            K = g_idx.numel()
             bits = _infer_bits(qweight, K)
             gs, gi = _group_layout(g_idx, K, scales.shape[1], perm)
             rows = gi is None and (_rows_op or _native_rows())
