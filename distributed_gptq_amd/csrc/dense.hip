@@ -25,11 +25,12 @@ namespace {
 //     under the last MFMAs.
 // The barriers are bare: the compiler's own would also wait for the copies.
 //
-// Bound by the matrix units at the power limit.  Measured (bf16, us): 8192^3
-// 728 (1511 TFLOP/s), 4096 x 4096 x 14336 305 (1579), 2048 x 28672 x 4096 415
-// (fp16 366).  On the way: 32-k stages (64-byte rows, half cache lines) with
-// 32x32 MFMAs 854 at 8192^3, with 16x16 MFMAs 810; the scalar address work
-// after a barrier instead of before it cost a tenth of a stage.
+// Bound by the matrix units at the power limit.  Measured alone (bf16 / fp16,
+// us): 8192^3 728 / 756 (1511 TFLOP/s in bf16), 4096 x 4096 x 14336 302 / 317
+// (1591), 2048 x 28672 x 4096 347 / 364 (1388).  On the way (bf16, 8192^3):
+// 32-k stages (64-byte rows, half cache lines) with 32x32 MFMAs 854, with 16x16
+// MFMAs 810; the scalar address work after a barrier instead of before it cost
+// a tenth of a stage.
 constexpr int kBK = 64;
 constexpr int kRowBytes = kBK * 2;
 constexpr int kTileM = 256;

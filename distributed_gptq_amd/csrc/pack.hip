@@ -135,7 +135,7 @@ __device__ __forceinline__ void dequant_pairs(const uint32_t (&w)[BITS], float z
 // the stores: a thread takes 8 codes of kDqRows rows, so that a wave's store
 // is 1 KB of consecutive bytes (16-bit outputs; with 32 codes a thread the
 // four 16-byte stores were 64 bytes apart between lanes and 28672 x 4096 to
-// bf16 took 94 us against 57, 297 MB moved), and the loads of all rows
+// bf16 took 94 us against 55-61, 297 MB moved), and the loads of all rows
 // are in flight together.
 constexpr int kDqRows = 4;
 
@@ -245,7 +245,9 @@ __global__ __launch_bounds__(256) void plane_flags_k(const void* __restrict__ sc
 // One workgroup per 64 output rows x 128 columns; thread t decodes the 32-code
 // chunk t / 64 of row t % 64 and the planes go through LDS ([column][row], so
 // the stores to it are 128 contiguous bytes a wave) to 16-byte stores of 128
-// contiguous bytes per column.  4096 x 14336, 4-bit: 63 us (264 MB moved).
+// contiguous bytes per column.  4096 x 14336, 4-bit: 66 us with plane_flags_k
+// (264 MB moved), 80 + 7 us in a training step, where the caches hold other
+// data.
 template <int BITS>
 __global__ __launch_bounds__(256) void dequant_planes_t_k(const uint8_t* __restrict__ packed,
                                                           const void* __restrict__ scales,

@@ -193,10 +193,10 @@ def _planes_backward(M: int, N: int, K: int, bits: int, dtype: torch.dtype, perm
     contraction takes the dense kernel 1.5 us a round (0.7 us a round of
     halves); codes of up to 4 bits take 2 planes, 8-bit codes 3, an fp16 grad
     twice that; the fp32 product runs at 130 TFLOP/s, and putting an act-order
-    weight into input order costs it 8 us per million weights.  Measured (4-bit
-    bf16, us, new / old): 4096 x 14336 M = 64 / 256 / 1024: 193 / 215 / 266
-    against 149 / 317 / 908; 8-bit 14336 x 4096 M = 512 / 1024: 625 / 625
-    against 589 / 967."""
+    weight into input order costs it 8 us per million weights.  Measured (us,
+    planes against product): 4-bit 4096 x 14336 M = 64 / 256 / 1024, bf16 179 /
+    202 / 257 against 137 / 306 / 903, fp16 250 / 261 / 416 against 131 / 307 /
+    903; 8-bit bf16 14336 x 4096 M = 512 / 1024: 611 / 611 against 570 / 968."""
     if N % 64 or K % 32 or max(M, K) > 1 << 24 or N > 1 << 20:  # the kernels' ranges
         return False
     rounds = _dense_rounds(M, K)
